@@ -77,12 +77,10 @@ bool q4mi_mmvq(uint32_t ty, const uint8_t *d_w, uint64_t nrows, uint64_t ncols,
 
 /* Size library scratch before any graph capture (src/q4.h:958). */
 void q4_hip_moe_scratch_warm(void);
-/* Drain the library stream and return the decode kernels' timeout word: 0
- * when every bounded in-kernel wait completed; otherwise a wait gave up and
- * the results of the decode calls since the last check are wrong (the bits
- * are described by q4mi_status_text, which also becomes q4mi_last_error()).
- * clear != 0 resets the word.  No reference counterpart (the reference's
- * kernels have no bounded waits). */
+/* Drain the library stream and return the kernels' status word: 0 when there
+ * is nothing to report, else the bits described by q4mi_status_text (which
+ * also becomes q4mi_last_error()).  clear != 0 resets the word.  No reference
+ * counterpart. */
 uint32_t q4mi_device_status(int clear);
 const char *q4mi_status_text(uint32_t bits);
 /* Copy the fp32 h = silu(gate.q8(x)) * (up.q8(x)) of the last decode call,

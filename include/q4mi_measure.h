@@ -19,8 +19,8 @@ extern "C" {
 /* Which launches of the decode pair run: 1 = gate/up only, 2 = down only,
  * 3 = both (default).  Lets a benchmark time each kernel alone. */
 void q4mi_moe_phases(int mask);
-/* Cap the decode kernels' LDS at `bytes` (0: all of it), so their LDS rings
- * get reused within a launch. */
+/* Accepted and without effect: the decode kernels hold their weights in
+ * registers and have no LDS ring to shorten. */
 void q4mi_moe_lds_cap(uint32_t bytes);
 /* One launch of an MFMA throughput probe on the library stream (kind 0:
  * int8 32x32x32, 1: fp16 32x32x16); *ops = the launch's ops, for a

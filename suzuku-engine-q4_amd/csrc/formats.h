@@ -227,6 +227,7 @@ struct FmtQ6K {
 
 
 // ------------------------------------------- IQ2_XXS, IQ2_XS, IQ3_XXS
+// (their groups are decoded from registers, moe_unit.h; here the LDS tables)
 // LDS: the grid as magnitude dwords and the 7-bit sign index -> two byte-mask
 // dwords table (the sign byte's bit 7 is the parity of the other seven).
 __device__ inline uint2 iqxx_sign_masks(uint32_t i) {
@@ -257,55 +258,14 @@ __device__ inline void iq2x_init(Iq2xLds<N> *t, const uint16_t *codes, uint32_t 
 }
 
 struct FmtIQ2XXS {
-    static constexpr uint32_t kType = Q4MI_T_IQ2_XXS;
-    static constexpr uint32_t kTabBytes = sizeof(Iq2xLds<256>);
-    static constexpr bool kTwo = false;
     __device__ static inline void init(void *tab, uint32_t tid, uint32_t n) {
         iq2x_init((Iq2xLds<256> *)tab, q4mi_iq2xxs_code_dev, tid, n);
-    }
-    __device__ static inline void decode(const void *tab, const uint8_t *lb, const uint32_t *lw,
-                                         uint32_t row, uint32_t g, WGroup &o) {
-        const Iq2xLds<256> *t = (const Iq2xLds<256> *)tab;
-        const uint32_t B = row + 66u * (g >> 3), ib = g & 7u;
-        o.d = q4mi_h2f(lds_u16_at(lb, B)) * 0.125f;
-        const uint32_t gi = lds_u32_at(lw, B + 2u + 8u * ib);
-        const uint32_t aux = lds_u32_at(lw, B + 6u + 8u * ib);
-        o.m1 = o.m2 = 2 * (int)(aux >> 28) + 1;
-#pragma unroll
-        for (int l = 0; l < 4; l++) {
-            const uint2 e = t->grid[(gi >> (8 * l)) & 0xffu];
-            const uint2 m = t->smask[(aux >> (7 * l)) & 127u];
-            o.w[2 * l] = q4mi_sign4(e.x, m.x);
-            o.w[2 * l + 1] = q4mi_sign4(e.y, m.y);
-        }
     }
 };
 
 struct FmtIQ2XS {
-    static constexpr uint32_t kType = Q4MI_T_IQ2_XS;
-    static constexpr uint32_t kTabBytes = sizeof(Iq2xLds<512>);
-    static constexpr bool kTwo = true;
     __device__ static inline void init(void *tab, uint32_t tid, uint32_t n) {
         iq2x_init((Iq2xLds<512> *)tab, q4mi_iq2xs_code_dev, tid, n);
-    }
-    __device__ static inline void decode(const void *tab, const uint8_t *lb, const uint32_t *lw,
-                                         uint32_t row, uint32_t g, WGroup &o) {
-        const Iq2xLds<512> *t = (const Iq2xLds<512> *)tab;
-        const uint32_t B = row + 74u * (g >> 3), ib = g & 7u;
-        o.d = q4mi_h2f(lds_u16_at(lb, B)) * 0.125f;
-        const uint32_t v01 = lds_u32_at(lw, B + 2u + 8u * ib);
-        const uint32_t v23 = lds_u32_at(lw, B + 6u + 8u * ib);
-        const uint32_t sc = lds_u8_at(lb, B + 66u + ib);
-        o.m1 = 2 * (int)(sc & 15u) + 1;
-        o.m2 = 2 * (int)(sc >> 4) + 1;
-#pragma unroll
-        for (int l = 0; l < 4; l++) {
-            const uint32_t v = ((l < 2 ? v01 : v23) >> (16 * (l & 1))) & 0xffffu;
-            const uint2 e = t->grid[v & 511u];
-            const uint2 m = t->smask[v >> 9];
-            o.w[2 * l] = q4mi_sign4(e.x, m.x);
-            o.w[2 * l + 1] = q4mi_sign4(e.y, m.y);
-        }
     }
 };
 
@@ -315,9 +275,6 @@ struct Iq3xxsLds {
 };
 
 struct FmtIQ3XXS {
-    static constexpr uint32_t kType = Q4MI_T_IQ3_XXS;
-    static constexpr uint32_t kTabBytes = sizeof(Iq3xxsLds);
-    static constexpr bool kTwo = false;
     __device__ static inline void init(void *tab, uint32_t tid, uint32_t n) {
         Iq3xxsLds *t = (Iq3xxsLds *)tab;
         for (uint32_t i = tid; i < 256; i += n) {
@@ -332,81 +289,6 @@ struct FmtIQ3XXS {
         }
         for (uint32_t i = tid; i < 128; i += n) t->smask[i] = iqxx_sign_masks(i);
     }
-    __device__ static inline void decode(const void *tab, const uint8_t *lb, const uint32_t *lw,
-                                         uint32_t row, uint32_t g, WGroup &o) {
-        const Iq3xxsLds *t = (const Iq3xxsLds *)tab;
-        const uint32_t B = row + 98u * (g >> 3), ib = g & 7u;
-        o.d = q4mi_h2f(lds_u16_at(lb, B)) * 0.25f;
-        const uint32_t q0 = lds_u32_at(lw, B + 2u + 8u * ib);
-        const uint32_t q1 = lds_u32_at(lw, B + 6u + 8u * ib);
-        const uint32_t aux = lds_u32_at(lw, B + 66u + 4u * ib);
-        o.m1 = o.m2 = 2 * (int)(aux >> 28) + 1;
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const uint32_t gb = ((k < 4 ? q0 : q1) >> (8 * (k & 3))) & 0xffu;
-            const uint2 m = t->smask[(aux >> (7 * (k >> 1))) & 127u];
-            o.w[k] = q4mi_sign4(t->grid[gb], (k & 1) ? m.y : m.x);
-        }
-    }
-};
-
-// ------------------------------------------------------------------ IQ4_XS
-struct FmtIQ4XS {
-    static constexpr uint32_t kType = Q4MI_T_IQ4_XS;
-    static constexpr uint32_t kTabBytes = 0;
-    static constexpr bool kTwo = false;
-    __device__ static inline void init(void *, uint32_t, uint32_t) {}
-    __device__ static inline void decode(const void *, const uint8_t *lb, const uint32_t *lw,
-                                         uint32_t row, uint32_t g, WGroup &o) {
-        const uint32_t B = row + 136u * (g >> 3), ib = g & 7u;
-        o.d = q4mi_h2f(lds_u16_at(lb, B));
-        const uint32_t sh = lds_u16_at(lb, B + 2u);
-        const uint32_t sl = lds_u8_at(lb, B + 4u + (ib >> 1));
-        const int ls = (int)(((sl >> (4 * (ib & 1u))) & 15u) | (((sh >> (2 * ib)) & 3u) << 4));
-        o.m1 = o.m2 = ls - 32;
-        uint32_t q[4];
-        lds_dwords(lw, B + 8u + 16u * ib, q);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            o.w[k] = iq4nl_map(q[k] & 0x0F0F0F0Fu);
-            o.w[k + 4] = iq4nl_map((q[k] >> 4) & 0x0F0F0F0Fu);
-        }
-    }
-};
-
-template <uint32_t TY>
-struct FmtOf;
-template <>
-struct FmtOf<Q4MI_T_IQ4_NL> {
-    using F = FmtIQ4NL;
-};
-template <>
-struct FmtOf<Q4MI_T_Q2_0> {
-    using F = FmtQ20;
-};
-template <>
-struct FmtOf<Q4MI_T_IQ2_S> {
-    using F = FmtIQ2S;
-};
-template <>
-struct FmtOf<Q4MI_T_Q6_K> {
-    using F = FmtQ6K;
-};
-template <>
-struct FmtOf<Q4MI_T_IQ2_XXS> {
-    using F = FmtIQ2XXS;
-};
-template <>
-struct FmtOf<Q4MI_T_IQ2_XS> {
-    using F = FmtIQ2XS;
-};
-template <>
-struct FmtOf<Q4MI_T_IQ3_XXS> {
-    using F = FmtIQ3XXS;
-};
-template <>
-struct FmtOf<Q4MI_T_IQ4_XS> {
-    using F = FmtIQ4XS;
 };
 
 }  // namespace q4mi

@@ -5,18 +5,16 @@
 namespace q4mi {
 
 // Measurement hook: bit 0 runs the gate/up launch, bit 1 the down launch
-// (default both).  Lets a benchmark time each kernel of the pair alone.
+// (default both).  Lets a benchmark time each kernel of the pair alone (a
+// down launch over device lists reads the last gate/up launch's plan).
 static int g_phases = 3;
-// LDS budget of a decode block (q4mi_moe_lds_cap lowers it for tests).
-static size_t g_lds_cap = 0;
-size_t lds_cap() { return g_lds_cap ? std::min(g_lds_cap, kLdsCap) : kLdsCap; }
 
 template <int NT>
 static bool run_nt(uint32_t ty_gu, uint32_t ty_dn, const MoeArgs &a, uint32_t nu_host) {
     if (g_phases & 1) {
-        const bool ok = ty_gu == Q4MI_T_IQ3_S ? gu_dispatch<Q4MI_T_IQ3_S, NT>(a, nu_host)
-                      : ty_gu == Q4MI_T_Q8_0  ? gu_dispatch<Q4MI_T_Q8_0, NT>(a, nu_host)
-                                              : moe_fmt_gu(ty_gu, NT, a, nu_host);
+        const bool ok = ty_gu == Q4MI_T_IQ3_S ? gu_dispatch<Q4MI_T_IQ3_S, NT>(a)
+                      : ty_gu == Q4MI_T_Q8_0  ? gu_dispatch<Q4MI_T_Q8_0, NT>(a)
+                                              : moe_fmt_gu(ty_gu, NT, a);
         if (!ok) return false;
     }
     if (!(g_phases & 2)) return true;
@@ -53,9 +51,6 @@ static bool shape_ok(uint32_t gt, uint32_t ut, uint32_t dt, uint32_t in_dim, uin
 }
 
 static Plan *g_plan = nullptr;   // a device-list call's plan, gate/up -> down
-#ifdef Q4MI_TRACE
-static unsigned long long *g_trace = nullptr;
-#endif
 
 bool moe_warm(uint32_t n_ff) {
     if (!g_plan && !lib_malloc((void **)&g_plan, sizeof(Plan))) {
@@ -123,20 +118,6 @@ static bool moe_run(const uint8_t *base, uint64_t stride, const ListSrc &src,
     a.src = src;
     a.hl = hl;
     a.gplan = work.h ? work.plan : g_plan;
-    // a producer publishes each chunk before issuing its next one: a copy
-    // issue stalls while the memory system is saturated, and publishing only
-    // after the next chunk's issue delayed the first chunk by microseconds
-    a.ahead = 1;
-    a.plan_in = (g_phases & 1) ? 1u : 0u;   // down follows this call's gate/up
-#ifdef Q4MI_TRACE
-    if (!work.h && !g_trace && hipMalloc(&g_trace, 2 * 4096 * 32 * 8) == hipSuccess)
-        (void)hipMemset(g_trace, 0, 2 * 4096 * 32 * 8);
-    a.trace = g_trace;
-    a.dbg = getenv("Q4MI_DBG") ? (uint32_t)atoi(getenv("Q4MI_DBG")) : 0u;
-#endif
-#if defined(Q4MI_TRACE) || defined(Q4MI_KNOBS)
-    if (getenv("Q4MI_AHEAD")) a.ahead = (uint32_t)atoi(getenv("Q4MI_AHEAD"));
-#endif
     const uint32_t nt = src.n_tok;
     if (nt == 1) return run_nt<1>(gt, dt, a, nu_host);
     if (nt == 2) return run_nt<2>(gt, dt, a, nu_host);
@@ -250,21 +231,9 @@ extern "C" {
  * down only, 3 = both. */
 void q4mi_moe_phases(int mask) { g_phases = mask & 3; }
 
-/* Measurement build only: cap the decode kernels' LDS at `bytes` (0: the
- * CU's 160 KB), so that their LDS rings are reused within a launch. */
-void q4mi_moe_lds_cap(uint32_t bytes) { g_lds_cap = bytes; }
-#endif
-
-#ifdef Q4MI_TRACE
-/* Trace build only: copy the phase timestamps [2 kernels][4096 blocks][32]
- * (wall clock, 100 MHz) of the last traced call to host memory, and clear
- * them. */
-bool q4mi_trace_read(unsigned long long *dst, uint64_t n) {
-    if (!g_trace || n > 2ull * 4096 * 32) return false;
-    if (hipDeviceSynchronize() != hipSuccess) return false;
-    if (hipMemcpy(dst, g_trace, n * 8, hipMemcpyDeviceToHost) != hipSuccess) return false;
-    return hipMemset(g_trace, 0, 2 * 4096 * 32 * 8) == hipSuccess;
-}
+/* Measurement build only: accepted and without effect (the decode kernels
+ * hold their weights in registers; there is no LDS ring to shorten). */
+void q4mi_moe_lds_cap(uint32_t bytes) { (void)bytes; }
 #endif
 
 /* Copy the fp32 h of the last decode call, [64 unique experts][8 tokens]
@@ -284,26 +253,16 @@ bool q4mi_moe_copy_h(float *d_dst, uint32_t n_ff) {
     return true;
 }
 
-/* Drain the library stream and read the decode kernels' timeout word (0:
- * every bounded wait completed; else the bits of q4mi_status_text).  A
- * non-zero word also becomes q4mi_last_error(); clear != 0 resets it. */
+/* Drain the library stream and read the kernels' status word (0: nothing to
+ * report; else the bits of q4mi_status_text).  A non-zero word also becomes
+ * q4mi_last_error(); clear != 0 resets it. */
 uint32_t q4mi_device_status(int clear) {
-    uint32_t v = 0;
-    if (hipStreamSynchronize(stream()) != hipSuccess ||
-        hipMemcpyFromSymbol(&v, HIP_SYMBOL(g_moe_status), sizeof v, 0,
-                            hipMemcpyDeviceToHost) != hipSuccess) {
+    if (hipStreamSynchronize(stream()) != hipSuccess) {
         set_error("q4mi_device_status: device not readable");
         return 0x80000000u;
     }
-    v |= moe_fmt_status(clear);
-    v |= mmq_status(clear);
+    const uint32_t v = mmq_status(clear);
     if (v) set_error("%s", q4mi_status_text(v));
-    if (v && clear) {
-        const uint32_t z = 0;
-        if (hipMemcpyToSymbol(HIP_SYMBOL(g_moe_status), &z, sizeof z, 0,
-                              hipMemcpyHostToDevice) != hipSuccess)
-            set_error("q4mi_device_status: reset failed");
-    }
     return v;
 }
 

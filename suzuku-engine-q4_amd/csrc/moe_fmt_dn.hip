@@ -28,14 +28,4 @@ bool moe_fmt_dn(uint32_t ty, int nt, const MoeArgs &a, uint32_t nu_host) {
     return false;
 }
 
-uint32_t moe_fmt_status_dn(int clear) {
-    uint32_t v = 0, w = 0;
-    if (hipMemcpyFromSymbol(&v, HIP_SYMBOL(g_moe_status), sizeof v, 0, hipMemcpyDeviceToHost) !=
-        hipSuccess)
-        return 0x80000000u;
-    if (v && clear)
-        (void)hipMemcpyToSymbol(HIP_SYMBOL(g_moe_status), &w, sizeof w, 0, hipMemcpyHostToDevice);
-    return v;
-}
-
 }  // namespace q4mi

@@ -1,0 +1,62 @@
+"""GPU parity of the register-held weight units of the decode and window
+kernels at the shapes where their lane layouts change or leave remainders
+(4 to 128 units per gate/up row, 4 to 16 per down row, output rows that do
+not fill the last block, lists of one entry and of nearly 64), and of the
+8-values-per-lane q8 quantizer's general path (groups of zeros, of products
+below the normal range, with a NaN), against the C oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from test_gpu_decode import dev, host
+from test_gpu_formats import check_tokens, packed_experts
+
+import q4mi
+from q4mi.synth import (T_IQ2_S, T_IQ2_XS, T_IQ2_XXS, T_IQ3_S, T_IQ3_XXS, T_IQ4_NL, T_IQ4_XS,
+                        T_Q2_0, T_Q8_0)
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(T_Q8_0, T_Q8_0, 256, 256), (T_Q8_0, T_Q2_0, 640, 640), (T_IQ3_S, T_IQ3_S, 512, 1024),
+          (T_IQ2_XS, T_IQ4_NL, 1024, 256), (T_IQ4_XS, T_Q8_0, 2560, 1024),
+          (T_IQ2_XXS, T_Q2_0, 4096, 640), (T_IQ3_XXS, T_IQ2_S, 8192, 512)]
+
+
+@pytest.mark.parametrize("tg,td,H,F", SHAPES)
+@pytest.mark.parametrize("n_tok,k", [(1, 1), (1, 40), (3, 5), (8, 7)])
+def test_units_layer(gpu, oracle, tg, td, H, F, n_tok, k):
+    E = 48
+    if H * F > 1 << 20:
+        E, k = 12, min(k, 12)
+    rng = np.random.default_rng(tg * 1000 + H + 10 * n_tok + k)
+    arena, stride, og, ou, od = packed_experts(rng, E, H, F, tg, td)
+    d_arena = dev(arena)
+    x = rng.standard_normal((n_tok, H)).astype(np.float32)
+    if n_tok == 3:            # groups the short quantizer forms do not take
+        x[0, :32] = 0.0
+        x[1, 32:64] *= np.float32(1e-36)
+        x[2, 70] = np.nan
+    ids = np.stack([rng.choice(E, k, replace=False) for _ in range(n_tok)]).astype(np.int32)
+    w = rng.random((n_tok, k)).astype(np.float32)
+    yo, h = oracle.moe_tokens(H, F, tg, td, arena, stride, x, ids, w, want_h=True)
+    P = q4mi.ptr
+    if n_tok == 1:
+        y = dev(np.zeros(H, np.float32))
+        i0, w0 = np.ascontiguousarray(ids[0]), np.ascontiguousarray(w[0])
+        q4mi.check(gpu.q4_hip_moe_exec(P(d_arena), stride, i0.ctypes.data_as(ctypes.c_void_p),
+                                       w0.ctypes.data_as(ctypes.c_void_p), k, tg, og, tg, ou, td,
+                                       od, P(dev(x[0])), None, None, None, P(y), F, H, H),
+                   "q4_hip_moe_exec")
+        got = host(y)[None]
+    else:
+        es = np.full((n_tok, 64), -1, np.int32)
+        ew = np.zeros((n_tok, 64), np.float32)
+        es[:, :k], ew[:, :k] = ids, w
+        y = dev(np.zeros((n_tok, H), np.float32))
+        q4mi.check(gpu.q4_hip_moe_exec_win(P(d_arena), stride, P(dev(es)), P(dev(ew)),
+                                           P(dev(np.full(n_tok, k, np.int32))), n_tok, tg, og, tg,
+                                           ou, td, od, P(dev(x)), None, P(y), F, H, H), "exec_win")
+        got = host(y)
+    ties = check_tokens(oracle, got, yo, h, ids, w, arena, stride, od, td, H, F)
+    assert ties <= max(1, n_tok // 2)
