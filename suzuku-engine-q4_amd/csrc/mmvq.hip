@@ -4,7 +4,10 @@
 // already-quantized activations and can export the per-group int32 sums.
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "mmvq_engine.h"
+#include "moe_unit.h"
 #include "q4mi_internal.h"
 
 namespace q4mi {
@@ -118,6 +121,222 @@ __global__ __launch_bounds__(NTHR) void mmvq_k(const uint8_t *__restrict__ W, ui
     Q4MI_GTR(6);
 }
 
+// The same products with the weights in registers (moe_unit.h), the kernel of
+// most calls (unit_ok).  What bounds it: up to about 20 MB the launch, its
+// prologue (codes and tables, 1.6 us) and the first loads' latency; above,
+// the L1 path and, at several tokens, the codes' LDS reads.  Tile kernel /
+// this one, us: IQ3_S 4096 x 4096 at 1 / 4 / 8 tokens 6.0 / 4.4, 13.3 / 6.1,
+// 12.2 / 8.9; IQ3_S 151936 x 2048 57.8 / 29.4, 58.9 / 47.1, 90.5 / 69.0.
+//
+// 1024-thread
+// blocks, each with a contiguous share of the rows; a wave's task
+// is RPW = 64 / LPR rows, LPR lanes per row with UPL units each, and its
+// registers are refilled with the next unit as soon as one is decoded.  The
+// block holds the tokens' q8 codes in LDS, quantized there from fp32 x (XF)
+// or laid out from xq / xd.  A row's sum does not depend on nt or XF.
+//
+// LDS (from offset 0): [tables] | x codes [NT][K] | x scales [NT][K/32]
+template <uint32_t TY, int NT, int LPR, int UPL, bool XF>
+__global__ __launch_bounds__(1024) void mmvq_u_k(const uint8_t *__restrict__ W, uint32_t rows,
+                                                 uint32_t rb, const float *__restrict__ xf,
+                                                 const int8_t *__restrict__ xq,
+                                                 const float *__restrict__ xd, uint32_t nt,
+                                                 float *__restrict__ y, float scale,
+                                                 int32_t *__restrict__ sums) {
+    using U = Unit<TY>;
+    constexpr uint32_t RPW = 64 / LPR, kUnits = LPR * UPL, K = 64 * kUnits, kOpt = 8 * kUnits;
+    constexpr uint32_t kNT = 1024, kNW = kNT / 64;
+    static_assert(UPL == 1 || !U::kEven || U::step(LPR) % 4 == 0, "units of a lane share their shifts");
+    extern __shared__ __align__(16) uint8_t smem[];
+    const LPtr tab = 0;
+    int8_t *lq = (int8_t *)(smem + U::kTabBytes);
+    float *ld = (float *)(lq + NT * K);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t no = nt * kOpt;
+    const uint32_t code = U::code(tid, kNT);
+    for (uint32_t i = tid; i < no; i += kNT) {
+        const uint32_t t = NT == 1 ? 0u : i / kOpt, o = i - t * kOpt;
+        if constexpr (XF) {
+            quant_oct<TY>(ld_oct(xf, i), o, kUnits, lq + t * K, ld + t * (K / 32));
+        } else {
+            *(uint2 *)(lq + t * K + code_at<TY>(o, kUnits)) = ((const uint2 *)xq)[i];
+            const uint32_t g = o >> 2;
+            if ((o & 3u) == 0)
+                ld[t * (K / 32) + 2u * group_unit<TY>(g) + group_half<TY>(g)] = xd[t * (K / 32) + g];
+        }
+    }
+    U::init(smem, code, tid, kNT);
+
+    // this lane's units within a task's rows (rows past the matrix repeat its
+    // last one)
+    const uint32_t li = lane % LPR, slot = lane / LPR;
+    const typename U::Offs of = U::offs(min(slot, rows - 1u) * rb, li);
+    const uint32_t PT = (rows + RPW - 1) / RPW, rlast = rows > RPW ? rows - RPW : 0u;
+    const uint32_t q = PT / gridDim.x, r = PT % gridDim.x, b = blockIdx.x;
+    const uint32_t T1 = b * q + min(b, r) + q + (b < r ? 1u : 0u);
+    uint32_t T = b * q + min(b, r) + wave;
+    constexpr int D = UPL > 1 ? 2 : 1;
+    typename U::Raw s[D];
+    uint32_t lT = T, lm = 0;      // next unit to load
+    GPtr lb = nullptr;
+    auto load = [&](typename U::Raw &s) __attribute__((always_inline)) {
+        const bool ok = lT < T1;
+        if (ok && (UPL == 1 || lm == 0)) lb = uniform_ptr(W + (uint64_t)min(lT * RPW, rlast) * rb);
+        U::load(s, lb + U::step(LPR) * lm, of, ok);
+        if (ok && ++lm == UPL) {
+            lm = 0;
+            lT += kNW;
+        }
+    };
+    if (T < T1) {
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+            load(s[k]);
+            asm volatile("" ::: "memory");
+        }
+    }
+    bar();
+    if (T >= T1) return;
+    // one or two tokens' codes of the lane's unit stay in registers
+    constexpr bool kXR = UPL == 1 && NT <= 2;
+    UnitX xr[kXR ? NT : 1];
+    if constexpr (kXR) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) load_unit_x(xr[t], lq + t * K, ld + t * (K / 32), kUnits, li);
+    }
+    // even and odd groups apart, so that a row's sum is the tile kernel's: its
+    // lanes hold one group each (two of them this lane's) and join pairs first
+    float acc[NT][2];
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[t][0] = acc[t][1] = 0.f;
+    uint32_t um = 0;
+    while (T < T1) {
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+            const uint32_t un = li + LPR * um;
+            const uint32_t row = min(T * RPW, rlast) + slot;
+            UnitW w;
+            if (k == 0 || T < T1) {
+                U::decode(tab, s[k], of, w);
+                if (!U::kRawW) unit_consumed(w);
+            }
+            if (!U::kRawW) load(s[k]);
+            if (k == 0 || T < T1) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    if (NT > 2 && (uint32_t)t >= nt) continue;
+                    UnitX xl;
+                    if constexpr (!kXR) load_unit_x(xl, lq + t * K, ld + t * (K / 32), kUnits, un);
+                    int sm[2];
+                    unit_dot2<TY>(w, kXR ? xr[kXR ? t : 0] : xl, acc[t], sm);
+                    if (!XF && sums && slot < rows) {
+                        int32_t *o = sums + ((size_t)t * rows + row) * (K / 32);
+                        o[unit_group<TY>(un, 0)] = sm[0];
+                        o[unit_group<TY>(un, 1)] = sm[1];
+                    }
+                }
+                if (UPL == 1 || ++um == UPL) {
+                    um = 0;
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        const float v = q4mi_rsum<LPR>(acc[t][1] + acc[t][0]);
+                        if (li == LPR - 1 && (uint32_t)t < nt && slot < rows)
+                            y[(size_t)t * rows + row] = scale * v;
+                        acc[t][0] = acc[t][1] = 0.f;
+                    }
+                    T += kNW;
+                }
+            }
+            if (U::kRawW) {
+                asm volatile("" ::: "memory");
+                load(s[k]);
+            }
+        }
+    }
+}
+
+template <uint32_t TY, int NT, int LPR, int UPL, bool XF>
+static bool unit_launch(const uint8_t *W, uint32_t rows, const float *xf, const int8_t *xq,
+                        const float *xd, uint32_t nt, float *y, float scale, int32_t *sums) {
+    constexpr uint32_t K = 64 * LPR * UPL, RPW = 64 / LPR;
+    const auto kern = mmvq_u_k<TY, NT, LPR, UPL, XF>;
+    static bool ready = false;
+    if (!ready) {
+        // the table lookups take the dynamic LDS to start at offset 0
+        hipFuncAttributes fa;
+        if (hipFuncGetAttributes(&fa, (const void *)kern) != hipSuccess || fa.sharedSizeBytes != 0 ||
+            hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                160 * 1024) != hipSuccess) {
+            set_error("mmvq: LDS limit");
+            return false;
+        }
+        ready = true;
+    }
+    const size_t lds = Unit<TY>::kTabBytes + (size_t)NT * K + (size_t)NT * (K / 32) * 4;
+    // one block per CU (each task at least one row set); the types without
+    // tables to build take up to four times as many for a tall matrix, which
+    // the CUs then share by their actual rate (Q8_0 151936 x 2048, 1 / 4
+    // tokens: 62.2 / 65.8 us with one block per CU, 57.8 / 64.5 with four)
+    const uint32_t tasks = (rows + RPW - 1) / RPW, cus = (uint32_t)cu_count();
+    const uint32_t most = Unit<TY>::kTabBytes ? 1u : 4u;
+    const uint32_t grid = std::min(cus * std::max(1u, std::min(most, tasks / (64u * cus))), tasks);
+    kern<<<dim3(grid), dim3(1024), lds, stream()>>>(W, rows, (uint32_t)q4mi_row_bytes(TY, K), xf, xq,
+                                                    xd, nt, y, scale, sums);
+    return launch_ok("mmvq_u_k");
+}
+
+template <uint32_t TY, int NT>
+static bool unit_nt(const uint8_t *W, uint32_t rows, uint32_t K, const float *xf, const int8_t *xq,
+                    const float *xd, uint32_t nt, float *y, float scale, int32_t *sums) {
+#define Q4MI_L(N, L, P)                                                                        \
+    case N:                                                                                    \
+        return xf ? unit_launch<TY, NT, L, P, true>(W, rows, xf, xq, xd, nt, y, scale, sums)   \
+                  : unit_launch<TY, NT, L, P, false>(W, rows, xf, xq, xd, nt, y, scale, sums);
+    switch (K / 64) {
+        // (Q8_0: twice the rows' groups per lane of the tile kernel's layout,
+        // whose sums it has to match)
+        Q4MI_L(4, 4, 1) Q4MI_L(8, 8, 1) Q4MI_L(16, 16, 1) Q4MI_L(32, 32, 1)
+        Q4MI_L(64, (TY == Q4MI_T_Q8_0 ? 32 : 64), (TY == Q4MI_T_Q8_0 ? 2 : 1))
+        Q4MI_L(128, (TY == Q4MI_T_Q8_0 ? 32 : 64), (TY == Q4MI_T_Q8_0 ? 4 : 2))
+        Q4MI_L(40, 8, 5)
+    case 10:   // 640 columns: not of the 256-value superblock types
+        if constexpr (TY == Q4MI_T_Q8_0 || TY == Q4MI_T_IQ4_NL || TY == Q4MI_T_Q2_0) {
+            return xf ? unit_launch<TY, NT, 2, 5, true>(W, rows, xf, xq, xd, nt, y, scale, sums)
+                      : unit_launch<TY, NT, 2, 5, false>(W, rows, xf, xq, xd, nt, y, scale, sums);
+        }
+    }
+#undef Q4MI_L
+    set_error("mmvq: K=%u not covered", K);
+    return false;
+}
+
+template <uint32_t TY>
+static bool unit_any(const uint8_t *W, uint32_t rows, uint32_t K, const float *xf, const int8_t *xq,
+                     const float *xd, uint32_t nt, float *y, float scale, int32_t *sums) {
+    if (nt == 1) return unit_nt<TY, 1>(W, rows, K, xf, xq, xd, nt, y, scale, sums);
+    if (nt == 2) return unit_nt<TY, 2>(W, rows, K, xf, xq, xd, nt, y, scale, sums);
+    if (nt <= 4) return unit_nt<TY, 4>(W, rows, K, xf, xq, xd, nt, y, scale, sums);
+    return unit_nt<TY, 8>(W, rows, K, xf, xq, xd, nt, y, scale, sums);
+}
+
+// Which kernel.  The register path takes rows that are whole dwords (others,
+// e.g. IQ3_S at 256 columns, keep the tile kernel's 2-byte copies), and is
+// the faster one over 480 calls (six types, 500-50000 rows, 1024-4096
+// columns, 1-8 tokens: 0.67 of the tile kernel's time in the geometric mean)
+// but for the tall Q8_0 matrices at one or two tokens, where the tile
+// kernel's many short blocks stream closer to the memory's rate.  Tile /
+// register kernel, us: 151936 x 2048 37.8 / 40.6 (1 token), 39.5 / 40.5 (2),
+// 49.7 / 44.2 (4); 70000 x 2048 19.5 / 19.7 and 20.8 / 20.3 (1, 2);
+// 151936 x 4096 83.4 / 80.8 (2).  The two give a row the same bits where
+// both take part (Q8_0), so a row's result still does not depend on nt.
+static bool unit_ok(uint32_t ty, const uint8_t *W, uint64_t rows, uint64_t K, uint32_t nt) {
+    const uint64_t rb = q4mi_row_bytes(ty, K), bytes = rows * rb;
+    if (((uintptr_t)W & 3u) || rb % 4) return false;
+    if (ty != Q4MI_T_Q8_0 || nt > 2) return true;
+    return nt == 1 ? bytes < (144ull << 20) : bytes < (160ull << 20) || K > 2560;
+}
+
 // weight bytes per row tile
 static uint32_t tile_target(uint32_t ty) {
     return ty == Q4MI_T_Q8_0 || ty == Q4MI_T_Q6_K ? 24576u : 14336u;
@@ -228,6 +447,16 @@ static bool mmvq_any(uint32_t ty, const uint8_t *W, uint64_t rows, uint64_t K, c
                      const int8_t *xq, const float *xd, uint32_t nt, float *y, float scale,
                      int32_t *sums) {
     const uint32_t r = (uint32_t)rows, k = (uint32_t)K;
+    if (unit_ok(ty, W, rows, K, nt)) {
+        switch (ty) {
+        case Q4MI_T_IQ3_S: return unit_any<Q4MI_T_IQ3_S>(W, r, k, xf, xq, xd, nt, y, scale, sums);
+        case Q4MI_T_Q8_0: return unit_any<Q4MI_T_Q8_0>(W, r, k, xf, xq, xd, nt, y, scale, sums);
+        case Q4MI_T_IQ4_NL: return unit_any<Q4MI_T_IQ4_NL>(W, r, k, xf, xq, xd, nt, y, scale, sums);
+        case Q4MI_T_Q2_0: return unit_any<Q4MI_T_Q2_0>(W, r, k, xf, xq, xd, nt, y, scale, sums);
+        case Q4MI_T_IQ2_S: return unit_any<Q4MI_T_IQ2_S>(W, r, k, xf, xq, xd, nt, y, scale, sums);
+        case Q4MI_T_Q6_K: return unit_any<Q4MI_T_Q6_K>(W, r, k, xf, xq, xd, nt, y, scale, sums);
+        }
+    }
     switch (ty) {
     case Q4MI_T_IQ3_S: return mmvq_launch<FmtIQ3S>(W, r, k, xf, xq, xd, nt, y, scale, sums);
     case Q4MI_T_Q8_0: return mmvq_launch<FmtQ80>(W, r, k, xf, xq, xd, nt, y, scale, sums);
@@ -245,8 +474,8 @@ bool mmvq_q8(uint32_t ty, const uint8_t *W, uint64_t rows, uint64_t K, const int
     return mmvq_any(ty, W, rows, K, nullptr, xq, xd, nt, y, scale, sums);
 }
 
-// Activations quantized inside the GEMV blocks: used while the codes of the
-// padded token count fit 16 KB of LDS beside the tile and the call has at
+// Activations quantized inside the tile kernel's blocks: used while the codes
+// of the padded token count fit 16 KB of LDS beside the tile and the call has at
 // most 1024 row tiles.  Every block re-reads and re-quantizes all of x, so
 // a tall matrix (config 4: 18992 tiles) is faster with one quantize launch
 // (measured: 56.5 against 70.8 us at 1 token), a short one (config 0: 512
@@ -312,7 +541,7 @@ bool q4_mmvq_n(uint32_t ty, const uint8_t *d_w, uint64_t nrows, uint64_t ncols,
         set_error("q4_mmvq_n: not covered");
         return false;
     }
-    if ((uintptr_t)d_x % 16 == 0 && mmvq_fused_fits(ty, nrows, ncols, n)) {
+    if ((uintptr_t)d_x % 16 == 0 && (unit_ok(ty, d_w, nrows, ncols, n) || mmvq_fused_fits(ty, nrows, ncols, n))) {
         // every block quantizes x itself: no quantize launch, no held codes
         g_cur_x = nullptr;
         return mmvq_f32(ty, d_w, nrows, ncols, d_x, n, d_y, scale);

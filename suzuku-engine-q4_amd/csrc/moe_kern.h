@@ -314,44 +314,6 @@ __host__ __device__ inline size_t al16(size_t v) { return (v + 15) & ~(size_t)15
 
 __device__ inline float silu_f(float v) { return v / (1.f + expf(-v)); }
 
-// Workgroup barrier without the compiler's fence: this wave's LDS operations
-// are complete, its loads from global memory stay in flight.
-__device__ inline void bar() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// ... and one for which this wave's loads are back too: issued before the
-// weight stream, so that no wave's weights queue ahead of another's inputs
-// (loads issued into the burst return when it drains).
-__device__ inline void bar_loads() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// Keep a uniform pointer one scalar register pair: the compiler otherwise
-// folds its terms into every lane address that is built on it.
-__device__ inline GPtr uniform_ptr(const uint8_t *p) {
-    uint64_t v = (uint64_t)p;
-    asm("" : "+s"(v));
-    return (GPtr)v;
-}
-
-// Between a unit's decode and the load that refills its registers: every
-// field is consumed (the table lookups are issued, multipliers and scales
-// formed) before the load, so the new values can take the same registers.
-__device__ inline void unit_consumed(UnitW &w) {
-    asm volatile("" : "+v"(w.m[0]), "+v"(w.m[1]), "+v"(w.m[2]), "+v"(w.m[3]), "+v"(w.d[0]),
-                 "+v"(w.d[1]) :: "memory");
-}
-
-// q8 of oct i (values 8i..8i+7) of a run of 32-value groups, codes laid out
-// by units (code_at, nu units): the 4 lanes holding octs 4g..4g+3 quantize
-// group g together (all 4 must be active).
-struct Oct { float4 x, y; };
-__device__ inline Oct ld_oct(const float *p, uint32_t i) {
-    return Oct{((const float4 *)p)[2 * i], ((const float4 *)p)[2 * i + 1]};
-}
-__device__ inline void quant_oct(const Oct &v, uint32_t i, uint32_t nu, int8_t *q, float *d) {
-    float dd;
-    *(uint2 *)(q + code_at(i, nu)) = q4mi_quant_team4(v.x, v.y, &dd);
-    if ((i & 3u) == 0) d[i / 4] = dd;
-}
-
 // ------------------------------------------------------------- gate / up
 // What bounds it: a one-token launch (hidden 2048, 11 experts, 9.9 MB) is the
 // launch itself (1.7 us), the prologue (activations in, q8 codes and tables

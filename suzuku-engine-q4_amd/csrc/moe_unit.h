@@ -492,32 +492,108 @@ struct Unit<Q4MI_T_IQ4_XS> {
     }
 };
 
+// -------------------------------------------------------------------- Q6_K
+// A unit is groups 4h + b and 4h + b + 2 of a superblock (half h, b = 0, 1):
+// the low and the high nibbles of the same 32 ql bytes, with two bits each of
+// the same 32 qh bytes.
+template <>
+struct Unit<Q4MI_T_Q6_K> {
+    static constexpr uint32_t kTabBytes = 0;
+    static constexpr bool kTwo = true;
+    static constexpr int kRegs = 21;
+    static constexpr bool kRawW = false;
+    struct Offs { uint32_t ql, qh, sc, d, s, ss, b; };
+    struct Raw { u32x4_t l[2], h[2]; uint32_t l8, h8; u32x2_t sc; uint32_t d; };
+    __device__ static inline Offs offs(uint32_t row, uint32_t u) {
+        const uint32_t p = row + (u >> 2) * 210u, h = (u >> 1) & 1u, b = u & 1u;
+        const uint32_t ql = p + 64u * h + 32u * b, qh = p + 128u + 32u * h,
+                       sc = p + 192u + 8u * h + 2u * b;
+        // (at shift 0 the ninth dwords are not needed; an odd superblock, the
+        // row's last among them, sits 2 bytes into its dwords)
+        return Offs{ql & ~3u, qh & ~3u, sc & ~3u, (p + 208u) & ~3u, p & 3u, 8u * (sc & 3u), b};
+    }
+    static constexpr uint32_t step(uint32_t n) { return n / 4 * 210u; }
+    static constexpr bool kEven = true;
+    __device__ static inline void load(Raw &r, GPtr b, const Offs &o, bool ok) {
+        r.l[0] = ld4_at<u32x4_t>(b, o.ql, ok);
+        r.l[1] = ld4_at<u32x4_t>(b, o.ql, ok, 16u);
+        r.l8 = ld4_at<uint32_t>(b, o.ql, ok, 32u);
+        r.h[0] = ld4_at<u32x4_t>(b, o.qh, ok);
+        r.h[1] = ld4_at<u32x4_t>(b, o.qh, ok, 16u);
+        r.h8 = ld4_at<uint32_t>(b, o.qh, ok, 32u);
+        r.sc = ld4_at<u32x2_t>(b, o.sc, ok);
+        r.d = ld4_at<uint32_t>(b, o.d, ok);
+    }
+    __device__ static inline uint32_t code(uint32_t, uint32_t) { return 0; }
+    __device__ static inline void init(void *, uint32_t, uint32_t, uint32_t) {}
+    __device__ static inline void decode(LPtr, const Raw &r, const Offs &f, UnitW &o) {
+        o.d[0] = o.d[1] = q4mi_h2f(r.d >> (8u * f.s));
+        // scales sc[8h + 2b], +1 (values 0-15, 16-31) and 4 later
+        const uint32_t s0 = r.sc.x >> f.ss, s1 = r.sc.y >> f.ss;
+        o.m[0] = (int)(int8_t)(s0 & 0xffu);
+        o.m[1] = (int)(int8_t)((s0 >> 8) & 0xffu);
+        o.m[2] = (int)(int8_t)(s1 & 0xffu);
+        o.m[3] = (int)(int8_t)((s1 >> 8) & 0xffu);
+        const uint32_t l[9] = {r.l[0].x, r.l[0].y, r.l[0].z, r.l[0].w, r.l[1].x, r.l[1].y, r.l[1].z, r.l[1].w, r.l8};
+        const uint32_t h[9] = {r.h[0].x, r.h[0].y, r.h[0].z, r.h[0].w, r.h[1].x, r.h[1].y, r.h[1].z, r.h[1].w, r.h8};
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t ql = __builtin_amdgcn_alignbyte(l[k + 1], l[k], f.s);
+            const uint32_t qh = __builtin_amdgcn_alignbyte(h[k + 1], h[k], f.s) >> (2u * f.b);
+            o.w[k] = q6_sub32((ql & 0x0F0F0F0Fu) | ((qh & 0x03030303u) << 4));
+            o.w[8 + k] = q6_sub32(((ql >> 4) & 0x0F0F0F0Fu) | (qh & 0x30303030u));
+        }
+    }
+};
+
+// Which unit and half holds group g of a row, and back.
+template <uint32_t TY>
+__device__ inline uint32_t group_unit(uint32_t g) {
+    return TY == Q4MI_T_Q6_K ? (g >> 2) * 2u + (g & 1u) : g >> 1;
+}
+template <uint32_t TY>
+__device__ inline uint32_t group_half(uint32_t g) {
+    return TY == Q4MI_T_Q6_K ? (g >> 1) & 1u : g & 1u;
+}
+template <uint32_t TY>
+__device__ inline uint32_t unit_group(uint32_t u, uint32_t half) {
+    return TY == Q4MI_T_Q6_K ? (u >> 1) * 4u + (u & 1u) + 2u * half : 2u * u + half;
+}
+
 // q8 codes of a run of units in LDS: 16-byte chunk c (0..3) of unit u at
 // (c * nu + u) * 16, so that lanes holding consecutive units read
 // consecutive 16-byte words (a unit's 64 bytes side by side would put every
-// second lane on the same banks); group scales in natural order.
+// second lane on the same banks); group scales at 2 unit + half.
+template <uint32_t TY = 0>
 __device__ inline uint32_t code_at(uint32_t oct, uint32_t nu) {   // oct = 8 values
-    return (((oct >> 1) & 3u) * nu + (oct >> 3)) * 16u + (oct & 1u) * 8u;
+    const uint32_t g = oct >> 2, c = 2u * group_half<TY>(g) + ((oct >> 1) & 1u);
+    return (c * nu + group_unit<TY>(g)) * 16u + (oct & 1u) * 8u;
 }
 
 // The unit's value against one token: xq / xd = that token's codes (laid out
 // as above over nu units) and scales.
-template <uint32_t TY>
-__device__ inline float unit_dot(const UnitW &o, const int8_t *xq, const float *xd, uint32_t nu,
-                                 uint32_t u, float acc) {
+struct UnitX {
     int32_t q[16];
+    float2 d;
+};
+__device__ inline void load_unit_x(UnitX &x, const int8_t *xq, const float *xd, uint32_t nu,
+                                   uint32_t u) {
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         const int4 v = *(const int4 *)(xq + ((uint32_t)c * nu + u) * 16u);
-        q[4 * c] = v.x;
-        q[4 * c + 1] = v.y;
-        q[4 * c + 2] = v.z;
-        q[4 * c + 3] = v.w;
+        x.q[4 * c] = v.x;
+        x.q[4 * c + 1] = v.y;
+        x.q[4 * c + 2] = v.z;
+        x.q[4 * c + 3] = v.w;
     }
-    const float2 dx = *(const float2 *)(xd + 2u * u);
+    x.d = *(const float2 *)(xd + 2u * u);
+}
+// The two groups' exact sums s, and their values added to acc[0] and acc[1].
+template <uint32_t TY>
+__device__ inline void unit_dot2(const UnitW &o, const UnitX &x, float (&acc)[2], int (&s)[2]) {
+    const auto &q = x.q;
     // exact group sums (24-bit multiplies, full rate: |sums| < 2^20,
     // |multipliers| <= 2^7)
-    int s[2];
 #pragma unroll
     for (int g = 0; g < 2; g++) {
         int a = 0;
@@ -534,8 +610,53 @@ __device__ inline float unit_dot(const UnitW &o, const int8_t *xq, const float *
             s[g] = __mul24(a, o.m[2 * g]);
         }
     }
-    acc = fmaf((float)s[0], o.d[0] * dx.x, acc);
-    return fmaf((float)s[1], o.d[1] * dx.y, acc);
+    acc[0] = fmaf((float)s[0], o.d[0] * x.d.x, acc[0]);
+    acc[1] = fmaf((float)s[1], o.d[1] * x.d.y, acc[1]);
+}
+template <uint32_t TY>
+__device__ inline float unit_dot(const UnitW &o, const int8_t *xq, const float *xd, uint32_t nu,
+                                 uint32_t u, float acc) {
+    UnitX x;
+    load_unit_x(x, xq, xd, nu, u);
+    int s[2];
+    float a[2] = {acc, 0.f};
+    unit_dot2<TY>(o, x, a, s);
+    return a[1] + a[0];
+}
+
+// Workgroup barrier without the compiler's fence: this wave's LDS operations
+// are complete, its loads from global memory stay in flight.
+__device__ inline void bar() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Keep a uniform pointer one scalar register pair: the compiler otherwise
+// folds its terms into every lane address that is built on it.
+__device__ inline GPtr uniform_ptr(const uint8_t *p) {
+    uint64_t v = (uint64_t)p;
+    asm("" : "+s"(v));
+    return (GPtr)v;
+}
+
+// Between a unit's decode and the load that refills its registers: every
+// field is consumed (the table lookups are issued, multipliers and scales
+// formed) before the load, so the new values can take the same registers.
+__device__ inline void unit_consumed(UnitW &w) {
+    asm volatile("" : "+v"(w.m[0]), "+v"(w.m[1]), "+v"(w.m[2]), "+v"(w.m[3]), "+v"(w.d[0]),
+                 "+v"(w.d[1]) :: "memory");
+}
+
+// q8 of oct i (values 8i..8i+7) of a row of 32-value groups, codes laid out by
+// the row's nu units: the 4 lanes holding octs 4g..4g+3 quantize group g
+// together (all 4 must be active).
+struct Oct { float4 x, y; };
+__device__ inline Oct ld_oct(const float *p, uint32_t i) {
+    return Oct{((const float4 *)p)[2 * i], ((const float4 *)p)[2 * i + 1]};
+}
+template <uint32_t TY = 0>
+__device__ inline void quant_oct(const Oct &v, uint32_t i, uint32_t nu, int8_t *q, float *d) {
+    float dd;
+    *(uint2 *)(q + code_at<TY>(i, nu)) = q4mi_quant_team4(v.x, v.y, &dd);
+    const uint32_t g = i >> 2;
+    if ((i & 3u) == 0) d[2u * group_unit<TY>(g) + group_half<TY>(g)] = dd;
 }
 
 }  // namespace q4mi

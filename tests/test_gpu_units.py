@@ -1,5 +1,5 @@
-"""GPU parity of the register-held weight units of the decode and window
-kernels at the shapes where their lane layouts change or leave remainders
+"""GPU parity of the register-held weight units (decode, window and GEMV
+kernels) at the shapes where their lane layouts change or leave remainders
 (4 to 128 units per gate/up row, 4 to 16 per down row, output rows that do
 not fill the last block, lists of one entry and of nearly 64), and of the
 8-values-per-lane q8 quantizer's general path (groups of zeros, of products
@@ -14,7 +14,7 @@ from test_gpu_formats import check_tokens, packed_experts
 
 import q4mi
 from q4mi.synth import (T_IQ2_S, T_IQ2_XS, T_IQ2_XXS, T_IQ3_S, T_IQ3_XXS, T_IQ4_NL, T_IQ4_XS,
-                        T_Q2_0, T_Q8_0)
+                        T_Q2_0, T_Q6_K, T_Q8_0)
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +60,58 @@ def test_units_layer(gpu, oracle, tg, td, H, F, n_tok, k):
         got = host(y)
     ties = check_tokens(oracle, got, yo, h, ids, w, arena, stride, od, td, H, F)
     assert ties <= max(1, n_tok // 2)
+
+
+@pytest.mark.parametrize("K", [1024, 2048, 2560, 4096])
+def test_tall_q80_same_bits_for_every_token_count(gpu, K):
+    """A tall Q8_0 matrix: one and two tokens may take the tile kernel, more
+    the register kernel; a row's bits do not depend on it."""
+    import torch
+    from q4mi import synth
+    rows = (170 << 20) // (K // 32 * 34) + 3
+    w = synth.device_q80(rows * (K // 32 * 34), seed=K)
+    x = torch.randn((3, K), device="cuda", generator=torch.Generator("cuda").manual_seed(K))
+    ys = []
+    for n in (1, 2, 3):
+        y = torch.empty((n, rows), device="cuda")
+        gpu.q4_mmvq_warm()
+        q4mi.check(gpu.q4_mmvq_n(T_Q8_0, q4mi.ptr(w), rows, K, q4mi.ptr(x), q4mi.ptr(y), 0.5, n),
+                   "q4_mmvq_n")
+        ys.append(y)
+    assert torch.equal(ys[0][0], ys[2][0])
+    assert torch.equal(ys[1][1], ys[2][1])
+
+
+@pytest.mark.parametrize("ty", [T_IQ3_S, T_Q8_0, T_IQ4_NL, T_Q2_0, T_IQ2_S, T_Q6_K])
+@pytest.mark.parametrize("rows,K", [(1, 512), (3, 8192), (515, 1024), (517, 2560), (66, 4096)])
+def test_units_gemv(gpu, oracle, ty, rows, K):
+    """Row counts around a wave's task and lane layouts of 8 to 128 units:
+    group sums bit-exact, y to 1e-3, the fp32-x entry the same bits as the
+    pre-quantized one, a row the same for 1 and 5 tokens."""
+    import torch
+    from test_gpu_decode import empty
+    from conftest import rel_err
+    from q4mi import synth
+    rng = np.random.default_rng(ty + rows + K)
+    w = synth.matrix(rng, ty, rows, K)
+    x = rng.standard_normal((5, K)).astype(np.float32)
+    q, d = (np.stack([oracle.quant8(x[t])[i] for t in range(5)]) for i in (0, 1))
+    dw, P, bits = dev(w), q4mi.ptr, []
+    gpu.q4_mmvq_warm()
+    for n in (5, 1):
+        y, s = empty((n, rows), torch.float32), empty((n, rows, K // 32), torch.int32)
+        q4mi.check(gpu.q4mi_mmvq(ty, P(dw), rows, K, P(dev(q)), P(dev(d)), n, P(y), 1.0, P(s)),
+                   "q4mi_mmvq")
+        y2 = empty((n, rows), torch.float32)
+        q4mi.check(gpu.q4_mmvq_n(ty, P(dw), rows, K, P(dev(x)), P(y2), 1.0, n), "q4_mmvq_n")
+        assert np.array_equal(host(y).view(np.uint32), host(y2).view(np.uint32))
+        bits.append(host(y)[0].view(np.uint32))
+        if n == 5:
+            sums = host(s)
+            rb = w.size // rows
+            for t in (0, 4):
+                for r in {0, rows // 2, rows - 1}:
+                    want = oracle.group_sums(ty, w[r * rb:(r + 1) * rb], K, q[t])
+                    assert np.array_equal(sums[t, r], want), (t, r)
+            assert rel_err(host(y), oracle.dot8_rows(ty, w, rows, K, x)) <= 1e-3
+    assert np.array_equal(bits[0], bits[1])
