@@ -312,7 +312,27 @@ __device__ inline float host_weights(KArgs ka, uint32_t n) {
 
 __host__ __device__ inline size_t al16(size_t v) { return (v + 15) & ~(size_t)15; }
 
-__device__ inline float silu_f(float v) { return v / (1.f + expf(-v)); }
+// silu(g) * u in fp64: 2^f on [-1/2, 1/2] by its Taylor series in f ln 2 to
+// the tenth power (error below 3e-13), the reciprocal by one Newton step on
+// the hardware's.
+__device__ inline double silu_mul(double g, double u) {
+    const double t = fmin(fmax(g * -1.4426950408889634, -1100.0), 1100.0);
+    const double n = rint(t), x = (t - n) * 0.6931471805599453;
+    double p = 1.0 / 3628800;
+    p = fma(p, x, 1.0 / 362880);
+    p = fma(p, x, 1.0 / 40320);
+    p = fma(p, x, 1.0 / 5040);
+    p = fma(p, x, 1.0 / 720);
+    p = fma(p, x, 1.0 / 120);
+    p = fma(p, x, 1.0 / 24);
+    p = fma(p, x, 1.0 / 6);
+    p = fma(p, x, 0.5);
+    p = fma(p, x, 1.0);
+    p = fma(p, x, 1.0);
+    const double d = 1.0 + ldexp(p, (int)n);
+    const double r0 = __builtin_amdgcn_rcp(d), r = fma(fma(-d, r0, 1.0), r0, r0);
+    return g * (d < __builtin_inf() ? r : 0.0) * u;
+}
 
 // ------------------------------------------------------------- gate / up
 // What bounds it: a one-token launch (hidden 2048, 11 experts, 9.9 MB) is the
@@ -324,6 +344,11 @@ __device__ inline float silu_f(float v) { return v / (1.f + expf(-v)); }
 // us, 4 tokens at hidden 2560 IQ2_S (43 MB) 24.6 / 19.8 us.
 // One block of 16 waves per CU: two blocks of 64-register waves repeat the
 // prologue and took 19.0 us for the 4-token launch.
+//
+// Sums and silu are taken in fp64, at fp32's instruction rate: h is then the
+// correctly rounded one but for about 1e-9 of it, so that its q8 codes in the
+// down launch, which an fp32 sum's error moves now and then (about one code in
+// 200,000), are those of exact arithmetic.
 //
 // A wave's task is RPW = 64 / LPR intermediate rows of one expert: LPR lanes
 // per row with UPL units each (unit li + LPR m), first the gate rows, then
@@ -373,7 +398,7 @@ __device__ inline void share_weighted(uint32_t sel, uint32_t nu, uint32_t tpe, u
 template <int NT, int RPW>
 struct GuOut {
     static constexpr uint32_t kCap = 64 + NT * RPW;
-    float g[kCap], u[kCap];
+    double g[kCap], u[kCap];
     uint32_t dst[kCap];
 };
 
@@ -388,7 +413,7 @@ __global__ __launch_bounds__(kT) void moe_gu_k(MoeArgs a) {
     Plan *P = (Plan *)(smem + U::kTabBytes);
     int8_t *xq = (int8_t *)(P + 1);
     constexpr uint32_t kUnits = LPR * UPL, K = 64 * kUnits;   // a row's units, columns
-    float *xd = (float *)(xq + NT * K);
+    double *xd = (double *)(xq + NT * K);
     auto *outs = (GuOut<NT, RPW> *)(xd + NT * (K / 32));
     const uint32_t tid = threadIdx.x, lane = tid & 63u, bid = blockIdx.x, nblk = gridDim.x;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -482,18 +507,17 @@ __global__ __launch_bounds__(kT) void moe_gu_k(MoeArgs a) {
     uint32_t cnt = 0;
     auto flush = [&]() __attribute__((always_inline)) {
         for (uint32_t i = lane; i < cnt; i += 64) {
-            const float g = out.g[i], u = out.u[i];
-            a.h[out.dst[i]] = silu_f(g) * u;
+            a.h[out.dst[i]] = (float)silu_mul(out.g[i], out.u[i]);
         }
         cnt = 0;
     };
-    auto finish = [&](uint32_t t0, uint32_t u, uint32_t sel, const float (&g)[NT],
-                      const float (&up)[NT]) __attribute__((always_inline)) {
+    auto finish = [&](uint32_t t0, uint32_t u, uint32_t sel, const double (&g)[NT],
+                      const double (&up)[NT]) __attribute__((always_inline)) {
         const uint32_t r = (t0 - u * a.tpe) * RPW + slot;
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             if (NT > 1 && !((sel >> t) & 1u)) continue;
-            const float gs = q4mi_rsum<LPR>(g[t]), us = q4mi_rsum<LPR>(up[t]);
+            const double gs = q4mi_rsum<LPR>(g[t]), us = q4mi_rsum<LPR>(up[t]);
             if (li == LPR - 1) {
                 out.g[cnt + slot] = gs;
                 out.u[cnt + slot] = us;
@@ -504,9 +528,9 @@ __global__ __launch_bounds__(kT) void moe_gu_k(MoeArgs a) {
         if (cnt >= 64) flush();
     };
     if (T < T1) {
-        float g[NT], acc[NT];
+        double g[NT], acc[NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) acc[t] = 0.f;
+        for (int t = 0; t < NT; t++) acc[t] = 0.0;
         uint32_t up = 0, um = 0;              // half, unit of the one to compute
         uint32_t u = __umulhi(T, a.tpe_inv);
         uint32_t sel = uniq ? 1u : (uint32_t)__builtin_amdgcn_readlane((int)selv, u);
@@ -521,7 +545,7 @@ __global__ __launch_bounds__(kT) void moe_gu_k(MoeArgs a) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
                 if (NT == 1 || ((sel >> t) & 1u))
-                    acc[t] = unit_dot<TY>(w, xq + t * K, xd + t * (2u * kUnits), kUnits, un, acc[t]);
+                    acc[t] = unit_dot64<TY>(w, xq + t * K, xd + t * (2u * kUnits), kUnits, un, acc[t]);
             if (U::kRawW) load();
             if (UPL == 1 || ++um == UPL) {
                 um = 0;
@@ -536,7 +560,7 @@ __global__ __launch_bounds__(kT) void moe_gu_k(MoeArgs a) {
                 }
                 up ^= 1u;
 #pragma unroll
-                for (int t = 0; t < NT; t++) acc[t] = 0.f;
+                for (int t = 0; t < NT; t++) acc[t] = 0.0;
             }
         }
     }
@@ -762,7 +786,7 @@ static bool launch_gu(const MoeArgs &a) {
     b.tpe = a.n_ff / RPW;
     b.tpe_inv = (uint32_t)((0x100000000ull + b.tpe - 1) / b.tpe);
     const size_t fixed = al16(Unit<TY>::kTabBytes + sizeof(Plan) + (size_t)NT * a.K +
-                              (size_t)NT * (a.K / 32) * 4);
+                              (size_t)NT * (a.K / 32) * 8);
     const size_t lds = fixed + std::max(sizeof(GuOut<NT, RPW>) * kW, kPlanTable);
     return moe_launch(moe_gu_k<TY, NT, LPR, UPL, SRC>, b, (uint32_t)cu_count(), lds, ready,
                       "moe_gu_k");

@@ -26,6 +26,7 @@
 //   Raw, load     the fields of one unit
 //   kRawW         the decoded quads are the loaded registers themselves (the
 //                 registers are free only after the dots)
+//   kOneD         both groups have the same scale
 //   decode        16 signed int8 quads (natural order), the multipliers of
 //                 quads 0-3, 4-7, 8-11, 12-15, and the two groups' scales:
 //                 group g's exact sum is m[2g] * dot(quads 8g..8g+3) +
@@ -96,6 +97,7 @@ template <>
 struct Unit<Q4MI_T_IQ3_S> {
     static constexpr uint32_t kTabBytes = 32768;
     static constexpr bool kTwo = false;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 9;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, sg, qh, sc, d, s, hs, ss; };
@@ -177,6 +179,7 @@ template <>
 struct Unit<Q4MI_T_Q8_0> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
+    static constexpr bool kOneD = false;
     static constexpr int kRegs = 17;
     static constexpr bool kRawW = true;
     struct Offs { uint32_t b; };
@@ -211,6 +214,7 @@ template <>
 struct Unit<Q4MI_T_IQ4_NL> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
+    static constexpr bool kOneD = false;
     static constexpr int kRegs = 9;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t b; };
@@ -247,6 +251,7 @@ template <>
 struct Unit<Q4MI_T_Q2_0> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 5;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t b, s; };
@@ -279,6 +284,7 @@ template <>
 struct Unit<Q4MI_T_IQ2_S> {
     static constexpr uint32_t kTabBytes = sizeof(Iq2sLds);
     static constexpr bool kTwo = true;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 7;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, sg, qh, sc, d, s, hs, ss; };
@@ -328,6 +334,7 @@ template <>
 struct Unit<Q4MI_T_IQ2_XXS> {
     static constexpr uint32_t kTabBytes = sizeof(Iq2xLds<256>);
     static constexpr bool kTwo = false;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 5;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, d, s; };
@@ -371,6 +378,7 @@ template <>
 struct Unit<Q4MI_T_IQ2_XS> {
     static constexpr uint32_t kTabBytes = sizeof(Iq2xLds<512>);
     static constexpr bool kTwo = true;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 6;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, sc, d, s, ss; };
@@ -413,6 +421,7 @@ template <>
 struct Unit<Q4MI_T_IQ3_XXS> {
     static constexpr uint32_t kTabBytes = sizeof(Iq3xxsLds);
     static constexpr bool kTwo = false;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 7;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, ax, d, s; };
@@ -460,6 +469,7 @@ template <>
 struct Unit<Q4MI_T_IQ4_XS> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 10;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, b, k; };
@@ -500,6 +510,7 @@ template <>
 struct Unit<Q4MI_T_Q6_K> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = true;
+    static constexpr bool kOneD = true;
     static constexpr int kRegs = 21;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t ql, qh, sc, d, s, ss, b; };
@@ -576,22 +587,24 @@ struct UnitX {
     int32_t q[16];
     float2 d;
 };
-__device__ inline void load_unit_x(UnitX &x, const int8_t *xq, const float *xd, uint32_t nu,
-                                   uint32_t u) {
+__device__ inline void load_unit_q(int32_t (&q)[16], const int8_t *xq, uint32_t nu, uint32_t u) {
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         const int4 v = *(const int4 *)(xq + ((uint32_t)c * nu + u) * 16u);
-        x.q[4 * c] = v.x;
-        x.q[4 * c + 1] = v.y;
-        x.q[4 * c + 2] = v.z;
-        x.q[4 * c + 3] = v.w;
+        q[4 * c] = v.x;
+        q[4 * c + 1] = v.y;
+        q[4 * c + 2] = v.z;
+        q[4 * c + 3] = v.w;
     }
+}
+__device__ inline void load_unit_x(UnitX &x, const int8_t *xq, const float *xd, uint32_t nu,
+                                   uint32_t u) {
+    load_unit_q(x.q, xq, nu, u);
     x.d = *(const float2 *)(xd + 2u * u);
 }
-// The two groups' exact sums s, and their values added to acc[0] and acc[1].
+// The two groups' exact integer sums.
 template <uint32_t TY>
-__device__ inline void unit_dot2(const UnitW &o, const UnitX &x, float (&acc)[2], int (&s)[2]) {
-    const auto &q = x.q;
+__device__ inline void unit_sums(const UnitW &o, const int32_t (&q)[16], int (&s)[2]) {
     // exact group sums (24-bit multiplies, full rate: |sums| < 2^20,
     // |multipliers| <= 2^7)
 #pragma unroll
@@ -610,6 +623,11 @@ __device__ inline void unit_dot2(const UnitW &o, const UnitX &x, float (&acc)[2]
             s[g] = __mul24(a, o.m[2 * g]);
         }
     }
+}
+// ... and their values added to acc[0] and acc[1].
+template <uint32_t TY>
+__device__ inline void unit_dot2(const UnitW &o, const UnitX &x, float (&acc)[2], int (&s)[2]) {
+    unit_sums<TY>(o, x.q, s);
     acc[0] = fmaf((float)s[0], o.d[0] * x.d.x, acc[0]);
     acc[1] = fmaf((float)s[1], o.d[1] * x.d.y, acc[1]);
 }
@@ -619,9 +637,24 @@ __device__ inline float unit_dot(const UnitW &o, const int8_t *xq, const float *
     UnitX x;
     load_unit_x(x, xq, xd, nu, u);
     int s[2];
-    float a[2] = {acc, 0.f};
-    unit_dot2<TY>(o, x, a, s);
-    return a[1] + a[0];
+    unit_sums<TY>(o, x.q, s);
+    acc = fmaf((float)s[0], o.d[0] * x.d.x, acc);
+    return fmaf((float)s[1], o.d[1] * x.d.y, acc);
+}
+// ... in fp64 (xd: the scales as fp64): every product exact, the sum rounded
+// far below fp32.  (fp64 multiply-adds run at fp32's rate here.)
+template <uint32_t TY>
+__device__ inline double unit_dot64(const UnitW &o, const int8_t *xq, const double *xd, uint32_t nu,
+                                    uint32_t u, double acc) {
+    int32_t q[16];
+    load_unit_q(q, xq, nu, u);
+    const double2 dx = *(const double2 *)(xd + 2u * u);
+    int s[2];
+    unit_sums<TY>(o, q, s);
+    if constexpr (Unit<TY>::kOneD)
+        return fma((double)o.d[0], fma((double)s[0], dx.x, (double)s[1] * dx.y), acc);
+    acc = fma((double)s[0], (double)o.d[0] * dx.x, acc);
+    return fma((double)s[1], (double)o.d[1] * dx.y, acc);
 }
 
 // Workgroup barrier without the compiler's fence: this wave's LDS operations
@@ -651,8 +684,8 @@ struct Oct { float4 x, y; };
 __device__ inline Oct ld_oct(const float *p, uint32_t i) {
     return Oct{((const float4 *)p)[2 * i], ((const float4 *)p)[2 * i + 1]};
 }
-template <uint32_t TY = 0>
-__device__ inline void quant_oct(const Oct &v, uint32_t i, uint32_t nu, int8_t *q, float *d) {
+template <uint32_t TY = 0, class D>
+__device__ inline void quant_oct(const Oct &v, uint32_t i, uint32_t nu, int8_t *q, D *d) {
     float dd;
     *(uint2 *)(q + code_at<TY>(i, nu)) = q4mi_quant_team4(v.x, v.y, &dd);
     const uint32_t g = i >> 2;

@@ -263,6 +263,25 @@ __device__ inline float q4mi_rsum(float v) {
     return v;
 }
 
+// The same over fp64 (each half moved by DPP, then one add).
+template <int CTRL, int ROWS>
+__device__ inline double q4mi_dpp_add64(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xF, true);
+    return v + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <int W>
+__device__ inline double q4mi_rsum(double v) {
+    v = q4mi_dpp_add64<0x111, 0xF>(v);
+    if (W >= 4) v = q4mi_dpp_add64<0x112, 0xF>(v);
+    if (W >= 8) v = q4mi_dpp_add64<0x114, 0xF>(v);
+    if (W >= 16) v = q4mi_dpp_add64<0x118, 0xF>(v);
+    if (W >= 32) v = q4mi_dpp_add64<0x142, 0xA>(v);
+    if (W >= 64) v = q4mi_dpp_add64<0x143, 0xC>(v);
+    return v;
+}
+
 // Inclusive prefix sum over the 64 lanes of a wave by DPP (row shifts 1, 2,
 // 4, 8 within each 16-lane row, then the row-15 and row-31 broadcasts carry
 // the earlier rows' totals forward).
