@@ -185,7 +185,7 @@ struct MmqFmt {
                                      : TY == Q4MI_T_IQ4_NL ? 256u
                                      : TY == Q4MI_T_Q2_0   ? 256u
                                                            : 1u;
-    static constexpr bool kHalves = TY == Q4MI_T_IQ3_S;   // decode_a's K order
+    static constexpr bool kHalves = TY == Q4MI_T_IQ3_S || TY == Q4MI_T_IQ2_S;   // decode_a's K order
     // byte offset of group j's scale inside the superblock, and its factor
     __device__ static inline uint32_t doff(uint32_t j) {
         return TY == Q4MI_T_Q8_0 ? 34u * j : TY == Q4MI_T_IQ4_NL ? 18u * j
@@ -204,8 +204,7 @@ struct MmqLds {
     _Float16 act[2][MMQ_MB][64];            // 32 KB; reused for the fused hand-off
     float dx[2][MMQ_MB][2];                 // group scales of each staged pair
     uint8_t raw[2][MMQ_NB][RawSpec<TY>::SS];  // raw weight bytes per superblock
-    uint2 g16[MmqFmt<TY>::kTab];            // decode table (MmqFmt)
-    uint2 sm16[16];                         // sign nibble -> fp16 sign masks
+    alignas(16) uint2 g16[MmqFmt<TY>::kTab];   // decode table (MmqFmt)
 };
 
 struct MmqArgs {
@@ -255,8 +254,8 @@ typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 // Lane's A operands of group j for one weight row: A0 = values 8kh..8kh+7,
 // A1 = values 16+8kh..16+8kh+7; with MmqFmt::kHalves A0 = values 16kh..16kh+7,
 // A1 = values 16kh+8..16kh+15 (the activation chunks are picked to match), so
-// that an IQ3_S lane's index bytes, ninth bits and signs are one contiguous
-// field each.  The loop is bound by vector instructions (two waves per SIMD:
+// that an IQ3_S or IQ2_S lane's index bytes, upper index bits and signs are one
+// contiguous field each.  The loop is bound by vector instructions (two waves per SIMD:
 // 128 scale FMAs and 78 decode instructions a 64-value stage at 128 tokens,
 // against 16 MFMAs), so the decode takes the fewest: four table addresses from
 // two words by byte permutes, signs by one shift and one bit select a pair
@@ -359,29 +358,34 @@ __device__ inline void decode_a(const MmqLds<TY> &L, const uint8_t *R, uint32_t 
         }
     } else if constexpr (TY == Q4MI_T_IQ2_S) {
         // group j: grid points l = 0..3 (8 values each), index qs[4j+l] with
-        // 2 bits of qh[j]; A0 = point kh (multiplier of values 0-15), A1 =
-        // point 2+kh (values 16-31).  The table holds each point's eight
-        // magnitudes as fp16; the sign masks come from the sign byte.
-        const uint32_t qs4 = lds_u16(R + 2 + 4 * j) | (lds_u16(R + 4 + 4 * j) << 16);
-        const uint32_t sg4 = lds_u16(R + 34 + 4 * j) | (lds_u16(R + 36 + 4 * j) << 16);
-        const uint32_t qh = R[66 + j], sc = R[74 + j];
-        auto point = [&](uint32_t l, uint32_t mult, half8_t &A) __attribute__((always_inline)) {
-            const uint32_t idx = ((qs4 >> (8 * l)) & 0xffu) | ((qh << (8 - 2 * l)) & 0x300u);
-            const uint2 g0 = L.g16[2 * idx], g1 = L.g16[2 * idx + 1];
-            const uint32_t sg = (sg4 >> (8 * l)) & 0xffu;
-            const uint2 m0 = L.sm16[sg & 15u], m1 = L.sm16[sg >> 4];
-            // XG: the multiplier becomes fp16(d / 8 * (2s+1) * kXgWs)
-            const float mf = XG ? q4mi_h2f(lds_u16(R)) * 0.125f * (float)mult * kXgWs
-                                : (float)mult;
-            const half2_t mm = {(_Float16)mf, (_Float16)mf};
-            const uint32_t o0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, g0.x ^ m0.x) * mm);
-            const uint32_t o1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, g0.y ^ m0.y) * mm);
-            const uint32_t o2 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, g1.x ^ m1.x) * mm);
-            const uint32_t o3 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, g1.y ^ m1.y) * mm);
-            A = __builtin_bit_cast(half8_t, make_uint4(o0, o1, o2, o3));
+        // 2 bits of qh[j].  This lane's are points 2kh and 2kh + 1, which
+        // share one multiplier; its 16 signs are one field.  The table holds
+        // a point's eight magnitudes as fp16.  Per group 16 shifts and bit
+        // selects for the signs in place of four reads of a sign table: the
+        // 1024-token fp16-activation layer with it 301 -> 270 us.
+        const uint32_t q2 = lds_u16(R + 2 + 4 * j + 2 * kh);
+        const uint32_t sg = lds_u16(R + 34 + 4 * j + 2 * kh);
+        const uint32_t qh = (uint32_t)R[66 + j] >> (4 * kh);
+        const uint32_t s = ((uint32_t)R[74 + j] >> (4 * kh)) & 15u;
+        // bit 15 - 2p up: value 2p's sign at bit 15, value 2p + 1's at 31
+        const uint32_t sgn = sg | (sg << 15);
+        _Float16 mh;
+        if constexpr (XG)   // fp16(d / 8 * (2s+1) * kXgWs)
+            mh = (_Float16)(q4mi_h2f(lds_u16(R)) * 0.125f * (float)(2u * s + 1u) * kXgWs);
+        else mh = (_Float16)(uint16_t)(2u * s + 1u);
+        const half2_t mm = {mh, mh};
+        auto pair = [&](uint32_t g, int p) __attribute__((always_inline)) {
+            const uint32_t v = (g & 0x7FFF7FFFu) | ((sgn << (15 - 2 * p)) & 0x80008000u);
+            return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) * mm);
         };
-        point(kh, 2u * (sc & 15u) + 1u, A0);
-        point(2 + kh, 2u * (sc >> 4) + 1u, A1);
+        auto point = [&](int l, half8_t &A) __attribute__((always_inline)) {
+            const uint32_t idx = ((q2 >> (8 * l)) & 0xffu) | ((qh << (8 - 2 * l)) & 0x300u);
+            const uint4 g = *(const uint4 *)&L.g16[2 * idx];
+            A = __builtin_bit_cast(half8_t, make_uint4(pair(g.x, 4 * l), pair(g.y, 4 * l + 1),
+                                                       pair(g.z, 4 * l + 2), pair(g.w, 4 * l + 3)));
+        };
+        point(0, A0);
+        point(1, A1);
     } else {
         // Q8_0 block j of the superblock: qs at 34j+2; values 8kh.. and 16+8kh..
         const uint8_t *qs = R + 34 * j + 2;
@@ -635,12 +639,6 @@ __device__ __attribute__((always_inline)) inline void mmq_tile(const MmqArgs a, 
         for (int jj = 0; jj < 4; jj++)
             h[jj] = __builtin_bit_cast(uint16_t, (_Float16)(float)((int)((tid >> (2 * jj)) & 3u) - 1));
         L.g16[tid] = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-    }
-    if (TY == Q4MI_T_IQ2_S && tid < 16) {   // sign nibble -> fp16 sign masks
-        uint32_t sgn[4];
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) sgn[jj] = ((tid >> jj) & 1u) ? 0x8000u : 0u;
-        L.sm16[tid] = make_uint2(sgn[0] | (sgn[1] << 16), sgn[2] | (sgn[3] << 16));
     }
     for (uint32_t s = 0; s < nst; s++) {
         const uint32_t sbi = s / SPS, q = s % SPS;
