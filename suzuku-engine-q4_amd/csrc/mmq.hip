@@ -185,7 +185,6 @@ struct MmqFmt {
                                      : TY == Q4MI_T_IQ4_NL ? 256u
                                      : TY == Q4MI_T_Q2_0   ? 256u
                                                            : 1u;
-    static constexpr bool kHalves = TY == Q4MI_T_IQ3_S || TY == Q4MI_T_IQ2_S;   // decode_a's K order
     // byte offset of group j's scale inside the superblock, and its factor
     __device__ static inline uint32_t doff(uint32_t j) {
         return TY == Q4MI_T_Q8_0 ? 34u * j : TY == Q4MI_T_IQ4_NL ? 18u * j
@@ -242,6 +241,11 @@ struct MmqArgs {
 #define MMQ_KO(a, bit) false
 #endif
 
+// decode_a's K order: 16 consecutive values per lane half.  Not in XG mode,
+// whose fp32 sums over the whole K keep the order they have.
+template <uint32_t TY, bool XG>
+constexpr bool mmq_halves = !XG && (TY == Q4MI_T_IQ3_S || TY == Q4MI_T_IQ2_S);
+
 // Slot of IQ3_S codebook entry i in g16 (decode_a's address order).
 __device__ inline uint32_t iq3s_slot(uint32_t i) {
     return ((i >> 3) & 31u) | ((i & 7u) << 5) | (i & 256u);
@@ -252,7 +256,7 @@ __device__ inline uint32_t lds_u16(const uint8_t *p) { return *(const uint16_t *
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
 // Lane's A operands of group j for one weight row: A0 = values 8kh..8kh+7,
-// A1 = values 16+8kh..16+8kh+7; with MmqFmt::kHalves A0 = values 16kh..16kh+7,
+// A1 = values 16+8kh..16+8kh+7; with mmq_halves A0 = values 16kh..16kh+7,
 // A1 = values 16kh+8..16kh+15 (the activation chunks are picked to match), so
 // that an IQ3_S or IQ2_S lane's index bytes, upper index bits and signs are one
 // contiguous field each.  The loop is bound by vector instructions (two waves per SIMD:
@@ -271,16 +275,18 @@ template <uint32_t TY, bool XG = false>
 __device__ inline void decode_a(const MmqLds<TY> &L, const uint8_t *R, uint32_t j,
                                 uint32_t kh, half8_t &A0, half8_t &A1) {
     if constexpr (TY == Q4MI_T_IQ3_S) {
-        // This lane's 16 values are entries 4kh..4kh+3 of four values each.
+        // This lane's 16 values are four entries of four values: 4kh..4kh+3
+        // (mmq_halves), or 2kh, 2kh+1, 4+2kh, 5+2kh.
+        constexpr bool H = mmq_halves<TY, XG>;
 #if defined(Q4MI_MMQ_KO) && ((Q4MI_MMQ_KO >> 9) & 1)
         const uint32_t lv = (uint32_t)(uintptr_t)R;
         const uint32_t q4 = lv * 7u + j, qh = (lv >> 3) & 0xffu, sg = (lv >> 5) & 0xffffu;
         const uint32_t sc = (lv >> 2) & 0xffu;
 #else
-        const uint8_t *qs = R + 2 + 8 * j + 4 * kh;
-        const uint32_t q4 = lds_u16(qs) | (lds_u16(qs + 2) << 16);   // index bytes
-        const uint32_t qh = R[66 + j];                               // ninth bits
-        const uint32_t sg = lds_u16(R + 74 + 4 * j + 2 * kh);        // value v: bit v
+        const uint8_t *qs = R + 2 + 8 * j + (H ? 4 : 2) * kh, *sp = R + 74 + 4 * j + (H ? 2 : 1) * kh;
+        const uint32_t q4 = lds_u16(qs) | (lds_u16(qs + (H ? 2 : 4)) << 16);   // index bytes
+        const uint32_t qh = R[66 + j];                                         // ninth bits
+        const uint32_t sg = H ? lds_u16(sp) : sp[0] | ((uint32_t)sp[2] << 8);  // value v: bit v
         const uint32_t sc = R[106 + (j >> 1)];
 #endif
         // Byte address of entry i in the table (slot order iq3s_slot): low
@@ -288,7 +294,9 @@ __device__ inline void decode_a(const MmqLds<TY> &L, const uint8_t *R, uint32_t 
         // = its lower three and the ninth bit.  The multiply spreads the
         // four ninth bits to the four bytes.
         const uint32_t lo = q4 & 0xF8F8F8F8u;
-        const uint32_t nb = __umul24((qh >> (4 * kh)) & 15u, 0x204081u) & 0x01010101u;
+        const uint32_t n2 = qh >> (2 * kh);
+        const uint32_t n4 = H ? (qh >> (4 * kh)) & 15u : (n2 & 3u) | ((n2 >> 2) & 12u);
+        const uint32_t nb = __umul24(n4, 0x204081u) & 0x01010101u;
         const uint32_t hi = (nb << 3) | (q4 & 0x07070707u);
         // bit 15 - 2p up: value 2p's sign at bit 15, value 2p + 1's at 31
         const uint32_t sgn = sg | (sg << 15);
@@ -358,34 +366,44 @@ __device__ inline void decode_a(const MmqLds<TY> &L, const uint8_t *R, uint32_t 
         }
     } else if constexpr (TY == Q4MI_T_IQ2_S) {
         // group j: grid points l = 0..3 (8 values each), index qs[4j+l] with
-        // 2 bits of qh[j].  This lane's are points 2kh and 2kh + 1, which
-        // share one multiplier; its 16 signs are one field.  The table holds
-        // a point's eight magnitudes as fp16.  Per group 16 shifts and bit
-        // selects for the signs in place of four reads of a sign table: the
-        // 1024-token fp16-activation layer with it 301 -> 270 us.
-        const uint32_t q2 = lds_u16(R + 2 + 4 * j + 2 * kh);
-        const uint32_t sg = lds_u16(R + 34 + 4 * j + 2 * kh);
-        const uint32_t qh = (uint32_t)R[66 + j] >> (4 * kh);
-        const uint32_t s = ((uint32_t)R[74 + j] >> (4 * kh)) & 15u;
+        // 2 bits of qh[j], one multiplier for points 0 and 1 and one for 2
+        // and 3.  This lane's are points 2kh and 2kh + 1 (mmq_halves), or kh and
+        // 2 + kh; its 16 signs are put into one field.  The table holds a
+        // point's eight magnitudes as fp16.  In place of four reads of a sign
+        // table (and, before, whole 32-bit fields joined per lane): the
+        // 1024-token fp16-activation layer with an IQ4_NL down 296 -> 272 us.
+        constexpr bool H = mmq_halves<TY, XG>;
+        const uint8_t *qs = R + 2 + 4 * j + (H ? 2 : 1) * kh, *sp = qs + 32;
+        const uint32_t q2 = H ? lds_u16(qs) : qs[0] | ((uint32_t)qs[2] << 8);
+        const uint32_t sg = H ? lds_u16(sp) : sp[0] | ((uint32_t)sp[2] << 8);
+        const uint32_t qh = (uint32_t)R[66 + j] >> ((H ? 4 : 2) * kh), sc = R[74 + j];
         // bit 15 - 2p up: value 2p's sign at bit 15, value 2p + 1's at 31
         const uint32_t sgn = sg | (sg << 15);
-        _Float16 mh;
-        if constexpr (XG)   // fp16(d / 8 * (2s+1) * kXgWs)
-            mh = (_Float16)(q4mi_h2f(lds_u16(R)) * 0.125f * (float)(2u * s + 1u) * kXgWs);
-        else mh = (_Float16)(uint16_t)(2u * s + 1u);
-        const half2_t mm = {mh, mh};
-        auto pair = [&](uint32_t g, int p) __attribute__((always_inline)) {
-            const uint32_t v = (g & 0x7FFF7FFFu) | ((sgn << (15 - 2 * p)) & 0x80008000u);
-            return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) * mm);
+        auto mult = [&](uint32_t s) __attribute__((always_inline)) {
+            _Float16 mh;
+            if constexpr (XG)   // fp16(d / 8 * (2s+1) * kXgWs)
+                mh = (_Float16)(q4mi_h2f(lds_u16(R)) * 0.125f * (float)(2u * s + 1u) * kXgWs);
+            else mh = (_Float16)(uint16_t)(2u * s + 1u);
+            return half2_t{mh, mh};
         };
-        auto point = [&](int l, half8_t &A) __attribute__((always_inline)) {
-            const uint32_t idx = ((q2 >> (8 * l)) & 0xffu) | ((qh << (8 - 2 * l)) & 0x300u);
+        auto point = [&](int l, half2_t mm, half8_t &A) __attribute__((always_inline)) {
+            auto pair = [&](uint32_t g, int p) __attribute__((always_inline)) {
+                const uint32_t v = (g & 0x7FFF7FFFu) | ((sgn << (15 - 2 * p)) & 0x80008000u);
+                return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) * mm);
+            };
+            const uint32_t idx = ((q2 >> (8 * l)) & 0xffu) | ((qh << (8 - (H ? 2 : 4) * l)) & 0x300u);
             const uint4 g = *(const uint4 *)&L.g16[2 * idx];
             A = __builtin_bit_cast(half8_t, make_uint4(pair(g.x, 4 * l), pair(g.y, 4 * l + 1),
                                                        pair(g.z, 4 * l + 2), pair(g.w, 4 * l + 3)));
         };
-        point(0, A0);
-        point(1, A1);
+        if constexpr (H) {
+            const half2_t mm = mult((sc >> (4 * kh)) & 15u);
+            point(0, mm, A0);
+            point(1, mm, A1);
+        } else {
+            point(0, mult(sc & 15u), A0);
+            point(1, mult(sc >> 4), A1);
+        }
     } else {
         // Q8_0 block j of the superblock: qs at 34j+2; values 8kh.. and 16+8kh..
         const uint8_t *qs = R + 34 * j + 2;
@@ -595,7 +613,7 @@ __device__ __attribute__((always_inline)) inline void mmq_tile(const MmqArgs a, 
 #pragma unroll
         for (uint32_t hf = 0; hf < 2; hf++) {
             // logical 16-byte chunk
-            const uint32_t c = 4 * gl + (MmqFmt<TY>::kHalves ? 2 * kh + hf : 2 * hf + kh);
+            const uint32_t c = 4 * gl + (mmq_halves<TY, XG> ? 2 * kh + hf : 2 * hf + kh);
             boff[gl][hf] = 2u * (l31 * KS + 8u * (c ^ (l31 & 7u)));
         }
     const uint32_t dxoff = 4u * l31 * GPS;
