@@ -52,8 +52,8 @@ def _link(objs, lib):
 
 def build_variant(lib, defines, verbose=False):
     """A measurement-build variant with extra preprocessor defines (e.g. the
-    MMQ timing knockouts, Q4MI_MMQ_KO=bits, or the decode phase trace,
-    Q4MI_TRACE) linked into `lib`; objects go to _build/<lib name>."""
+    MMQ timing knockouts, Q4MI_MMQ_KO=bits, or the tile GEMV phase trace,
+    Q4MI_GTRACE) linked into `lib`; objects go to _build/<lib name>."""
     tag = os.path.splitext(os.path.basename(lib))[0]
     odir = os.path.join(OBJ, tag)
     os.makedirs(odir, exist_ok=True)
