@@ -128,8 +128,7 @@ __global__ __launch_bounds__(NTHR) void mmvq_k(const uint8_t *__restrict__ W, ui
 // this one, us: IQ3_S 4096 x 4096 at 1 / 4 / 8 tokens 6.0 / 4.4, 13.3 / 6.1,
 // 12.2 / 8.9; IQ3_S 151936 x 2048 57.8 / 29.4, 58.9 / 47.1, 90.5 / 69.0.
 //
-// 1024-thread
-// blocks, each with a contiguous share of the rows; a wave's task
+// 1024-thread blocks, each with a contiguous share of the rows; a wave's task
 // is RPW = 64 / LPR rows, LPR lanes per row with UPL units each, and its
 // registers are refilled with the next unit as soon as one is decoded.  The
 // block holds the tokens' q8 codes in LDS, quantized there from fp32 x (XF)
