@@ -348,7 +348,8 @@ __device__ inline double silu_mul(double g, double u) {
 // Sums and silu are taken in fp64, at fp32's instruction rate: h is then the
 // correctly rounded one but for about 1e-9 of it, so that its q8 codes in the
 // down launch, which an fp32 sum's error moves now and then (about one code in
-// 200,000), are those of exact arithmetic.
+// 200,000), are those of exact arithmetic.  (The times above are with fp32 sums;
+// fp64 adds 0.2 us at one token and 0.3 to 0.9 at four.)
 //
 // A wave's task is RPW = 64 / LPR intermediate rows of one expert: LPR lanes
 // per row with UPL units each (unit li + LPR m), first the gate rows, then
