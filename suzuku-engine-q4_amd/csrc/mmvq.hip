@@ -5,6 +5,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "mmvq_engine.h"
 #include "moe_unit.h"
@@ -121,18 +122,48 @@ __global__ __launch_bounds__(NTHR) void mmvq_k(const uint8_t *__restrict__ W, ui
     Q4MI_GTR(6);
 }
 
+// a = {its lower half, b's lower half}, b = {a's upper half, its upper half}.
+template <class T>
+__device__ inline void swap_halves(T &a, T &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a),
+                                                    __builtin_bit_cast(uint32_t, b), false, false);
+    const uint32_t r0 = r[0], r1 = r[1];
+    a = __builtin_bit_cast(T, r0);
+    b = __builtin_bit_cast(T, r1);
+}
+// The sum of two neighbouring groups of a row, one pair per lane.
+template <uint32_t TY>
+__device__ inline float pair_sum(const float (&acc)[2], uint32_t li) {
+    if constexpr (TY != Q4MI_T_Q6_K) return acc[1] + acc[0];
+    // lanes 2k, 2k + 1 hold groups 4k, 4k + 2 and 4k + 1, 4k + 3
+    const float keep = li & 1u ? acc[1] : acc[0], give = li & 1u ? acc[0] : acc[1];
+    return keep + q4mi_team8_swap<0xB1>(give);
+}
+
 // The same products with the weights in registers (moe_unit.h), the kernel of
 // most calls (unit_ok).  What bounds it: up to about 20 MB the launch, its
 // prologue (codes and tables, 1.6 us) and the first loads' latency; above,
 // the L1 path and, at several tokens, the codes' LDS reads.  Tile kernel /
-// this one, us: IQ3_S 4096 x 4096 at 1 / 4 / 8 tokens 6.0 / 4.4, 13.3 / 6.1,
-// 12.2 / 8.9; IQ3_S 151936 x 2048 57.8 / 29.4, 58.9 / 47.1, 90.5 / 69.0.
+// this one, us: IQ3_S 4096 x 4096 at 1 / 4 / 8 tokens 5.7 / 4.2, 13.0 / 6.5,
+// 11.5 / 9.4; IQ3_S 151936 x 2048 58.7 / 29.6, 56.7 / 45.3, 91.2 / 66.5.
 //
 // 1024-thread blocks, each with a contiguous share of the rows; a wave's task
 // is RPW = 64 / LPR rows, LPR lanes per row with UPL units each, and its
 // registers are refilled with the next unit as soon as one is decoded.  The
 // block holds the tokens' q8 codes in LDS, quantized there from fp32 x (XF)
-// or laid out from xq / xd.  A row's sum does not depend on nt or XF.
+// or laid out from xq / xd.
+//
+// A row's sum is the tile kernel's, bit for bit (so it depends neither on nt
+// or XF nor on the weights' address): its lane i holds groups i, i + TPR, ...,
+// adds them in that order by fp32 multiply-adds, and the lanes are joined as a
+// tree over their index.  Here a lane's units hold two such chains, joined
+// first.  Rows of 128 and 256 groups (TPR = 64) over 64 lanes put a chain's
+// groups into lanes l and l + 32: the halves of the wave swap one unit group's
+// sum and scale each (kFold), so that the lower lanes hold the chains of the
+// first groups of units l, l + 32, ... and the upper ones those of the second.
+// A Q6_K unit's groups lie two apart, so neighbouring lanes exchange one chain
+// (pair_sum).  With a lane's own groups added first instead, IQ3_S at 4096
+// columns had 8.0e-8 of error against 64 bits, not 7.7e-8.
 //
 // The grid size is an argument: reading gridDim makes the runtime fill 248
 // bytes of hidden arguments at every launch (host time of a call, IQ3_S 1024 x
@@ -202,15 +233,25 @@ __global__ __launch_bounds__(1024) void mmvq_u_k(const uint8_t *__restrict__ W, 
     }
     bar();
     if (T >= T1) return;
+    constexpr bool kFold = LPR == 64;
+    // token t's codes of unit un (the lane's um-th) and the scales they go with
+    auto load_x = [&](UnitX &x, int t, uint32_t un, uint32_t um) __attribute__((always_inline)) {
+        load_unit_q(x.q, lq + t * K, kUnits, un);
+        const float *d = ld + t * (K / 32);
+        if constexpr (kFold) {
+            d += 2u * ((li & 31u) + 64u * um) + (li >> 5);
+            x.d = make_float2(d[0], d[64]);
+        } else {
+            x.d = *(const float2 *)(d + 2u * un);
+        }
+    };
     // one or two tokens' codes of the lane's unit stay in registers
     constexpr bool kXR = UPL == 1 && NT <= 2;
     UnitX xr[kXR ? NT : 1];
     if constexpr (kXR) {
 #pragma unroll
-        for (int t = 0; t < NT; t++) load_unit_x(xr[t], lq + t * K, ld + t * (K / 32), kUnits, li);
+        for (int t = 0; t < NT; t++) load_x(xr[t], t, li, 0);
     }
-    // even and odd groups apart, so that a row's sum is the tile kernel's: its
-    // lanes hold one group each (two of them this lane's) and join pairs first
     float acc[NT][2];
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[t][0] = acc[t][1] = 0.f;
@@ -224,6 +265,7 @@ __global__ __launch_bounds__(1024) void mmvq_u_k(const uint8_t *__restrict__ W, 
             if (k == 0 || T < T1) {
                 U::decode(tab, s[k], of, w);
                 if (!U::kRawW) unit_consumed(w);
+                if (kFold) swap_halves(w.d[0], w.d[1]);
             }
             if (!U::kRawW) load(s[k]);
             if (k == 0 || T < T1) {
@@ -231,9 +273,15 @@ __global__ __launch_bounds__(1024) void mmvq_u_k(const uint8_t *__restrict__ W, 
                 for (int t = 0; t < NT; t++) {
                     if (NT > 2 && (uint32_t)t >= nt) continue;
                     UnitX xl;
-                    if constexpr (!kXR) load_unit_x(xl, lq + t * K, ld + t * (K / 32), kUnits, un);
+                    if constexpr (!kXR) load_x(xl, t, un, um);
+                    const UnitX &x = kXR ? xr[kXR ? t : 0] : xl;
                     int sm[2];
-                    unit_dot2<TY>(w, kXR ? xr[kXR ? t : 0] : xl, acc[t], sm);
+                    unit_sums<TY>(w, x.q, sm);
+                    int c[2] = {sm[0], sm[1]};
+                    if (kFold) swap_halves(c[0], c[1]);
+                    float &a0 = acc[t][0], &a1 = acc[t][kFold ? 0 : 1];
+                    a0 = fmaf((float)c[0], w.d[0] * x.d.x, a0);
+                    a1 = fmaf((float)c[1], w.d[1] * x.d.y, a1);
                     if (!XF && sums && slot < rows) {
                         int32_t *o = sums + ((size_t)t * rows + row) * (K / 32);
                         o[unit_group<TY>(un, 0)] = sm[0];
@@ -244,7 +292,11 @@ __global__ __launch_bounds__(1024) void mmvq_u_k(const uint8_t *__restrict__ W, 
                     um = 0;
 #pragma unroll
                     for (int t = 0; t < NT; t++) {
-                        const float v = q4mi_rsum<LPR>(acc[t][1] + acc[t][0]);
+                        if (kFold) {
+                            acc[t][1] = acc[t][0];
+                            swap_halves(acc[t][0], acc[t][1]);
+                        }
+                        const float v = q4mi_rsum<kFold ? 32 : LPR>(pair_sum<TY>(acc[t], li));
                         if (li == LPR - 1 && (uint32_t)t < nt && slot < rows)
                             y[(size_t)t * rows + row] = scale * v;
                         acc[t][0] = acc[t][1] = 0.f;
@@ -293,22 +345,42 @@ static bool unit_launch(const uint8_t *W, uint32_t rows, const float *xf, const 
 template <uint32_t TY, int NT>
 static bool unit_nt(const uint8_t *W, uint32_t rows, uint32_t K, const float *xf, const int8_t *xq,
                     const float *xd, uint32_t nt, float *y, float scale, int32_t *sums) {
-#define Q4MI_L(N, L, P)                                                                        \
-    case N:                                                                                    \
-        return xf ? unit_launch<TY, NT, L, P, true>(W, rows, xf, xq, xd, nt, y, scale, sums)   \
+    const auto go = [&](auto lpr, auto upl) {
+        constexpr int L = decltype(lpr)::value, P = decltype(upl)::value;
+        return xf ? unit_launch<TY, NT, L, P, true>(W, rows, xf, xq, xd, nt, y, scale, sums)
                   : unit_launch<TY, NT, L, P, false>(W, rows, xf, xq, xd, nt, y, scale, sums);
+    };
+    // 4096 and 8192 columns: 64 lanes a row, or 32 with twice the units (the
+    // same bits).  64 give the waves more tasks and swap sums (kFold) per unit
+    // and token; 32 are faster from three tokens on where there are four (Q6_K,
+    // whose units take more registers: eight) rows a wave and more.  64 / 32
+    // lanes, us, 4 tokens at 4096 columns: IQ3_S 4096 rows 6.5 / 7.0, 16384 13.1
+    // / 13.2, 32768 21.8 / 20.5; Q2_0 16384 12.4 / 11.4; Q6_K 24576 22.7 / 23.8,
+    // 32768 30.8 / 29.5, 50000 46.1 / 43.0.  Q8_0 (no table, 68 bytes a unit)
+    // always takes 32.
+    constexpr bool kMay32 = TY == Q4MI_T_Q8_0 || NT > 2, kMay64 = TY != Q4MI_T_Q8_0;
+    const bool l32 = !kMay64 || rows >= (TY == Q4MI_T_Q6_K ? 32768u : 16384u);
+    using std::integral_constant;
+#define Q4MI_L(L, P) go(integral_constant<int, L>(), integral_constant<int, P>())
     switch (K / 64) {
-        // (Q8_0: twice the rows' groups per lane of the tile kernel's layout,
-        // whose sums it has to match)
-        Q4MI_L(4, 4, 1) Q4MI_L(8, 8, 1) Q4MI_L(16, 16, 1) Q4MI_L(32, 32, 1)
-        Q4MI_L(64, (TY == Q4MI_T_Q8_0 ? 32 : 64), (TY == Q4MI_T_Q8_0 ? 2 : 1))
-        Q4MI_L(128, (TY == Q4MI_T_Q8_0 ? 32 : 64), (TY == Q4MI_T_Q8_0 ? 4 : 2))
-        Q4MI_L(40, 8, 5)
+    case 4: return Q4MI_L(4, 1);
+    case 8: return Q4MI_L(8, 1);
+    case 16: return Q4MI_L(16, 1);
+    case 32: return Q4MI_L(32, 1);
+    case 64:
+        if constexpr (kMay32)
+            if (l32) return Q4MI_L(32, 2);
+        if constexpr (kMay64) return Q4MI_L(64, 1);
+        break;
+    case 128:
+        if constexpr (kMay32)
+            if (l32) return Q4MI_L(32, 4);
+        if constexpr (kMay64) return Q4MI_L(64, 2);
+        break;
+    case 40: return Q4MI_L(8, 5);
     case 10:   // 640 columns: not of the 256-value superblock types
-        if constexpr (TY == Q4MI_T_Q8_0 || TY == Q4MI_T_IQ4_NL || TY == Q4MI_T_Q2_0) {
-            return xf ? unit_launch<TY, NT, 2, 5, true>(W, rows, xf, xq, xd, nt, y, scale, sums)
-                      : unit_launch<TY, NT, 2, 5, false>(W, rows, xf, xq, xd, nt, y, scale, sums);
-        }
+        if constexpr (TY == Q4MI_T_Q8_0 || TY == Q4MI_T_IQ4_NL || TY == Q4MI_T_Q2_0)
+            return Q4MI_L(2, 5);
     }
 #undef Q4MI_L
     set_error("mmvq: K=%u not covered", K);

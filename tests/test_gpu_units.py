@@ -3,7 +3,9 @@ kernels) at the shapes where their lane layouts change or leave remainders
 (4 to 128 units per gate/up row, 4 to 16 per down row, output rows that do
 not fill the last block, lists of one entry and of nearly 64), and of the
 8-values-per-lane q8 quantizer's general path (groups of zeros, of products
-below the normal range, with a NaN), against the C oracle."""
+below the normal range, with a NaN), against the C oracle; the GEMV's tile
+kernel, which takes weights that are not whole dwords, and its bits against
+the register kernel's."""
 import ctypes
 
 import numpy as np
@@ -115,3 +117,85 @@ def test_units_gemv(gpu, oracle, ty, rows, K):
                     assert np.array_equal(sums[t, r], want), (t, r)
             assert rel_err(host(y), oracle.dot8_rows(ty, w, rows, K, x)) <= 1e-3
     assert np.array_equal(bits[0], bits[1])
+
+
+GEMV_TYPES = [T_IQ3_S, T_Q8_0, T_IQ4_NL, T_Q2_0, T_IQ2_S, T_Q6_K]
+
+
+def offset_dev(w, by):
+    """A device copy of w that starts `by` bytes into an allocation."""
+    import torch
+    b = torch.zeros(w.size + by, dtype=torch.uint8, device="cuda")
+    b[by:] = torch.from_numpy(w).cuda()
+    return b[by:]
+
+
+@pytest.mark.parametrize("ty", GEMV_TYPES)
+@pytest.mark.parametrize("rows,K", [(33, 256), (9, 640), (70, 512), (4100, 2048), (37, 2560),
+                                    (130, 4096), (35, 8192)])
+def test_gemv_weights_two_bytes_into_a_dword(gpu, oracle, ty, rows, K):
+    """Weights that start 2 bytes into a dword, and rows that are not whole
+    dwords (256 columns of the 256-value superblock types), take the tile
+    kernel: group sums bit-exact and y to 1e-3 against the oracle, fp32 x the
+    same bits as pre-quantized codes, and the same bits as the register kernel
+    gives the same rows where their start is a whole dword."""
+    import torch
+    from test_gpu_decode import empty
+    from conftest import rel_err
+    from q4mi import synth
+    if K == 640 and ty in (T_IQ3_S, T_IQ2_S, T_Q6_K):
+        pytest.skip("not a whole number of superblocks")
+    rng = np.random.default_rng(ty + rows + K)
+    w = synth.matrix(rng, ty, rows, K)
+    x = rng.standard_normal((8, K)).astype(np.float32)
+    q, d = (np.stack([oracle.quant8(x[t])[i] for t in range(8)]) for i in (0, 1))
+    P, bases = q4mi.ptr, [offset_dev(w, 2), offset_dev(w, 0)]
+    dx, dq, dd = dev(x), dev(q), dev(d)
+    rb = w.size // rows
+    gpu.q4_mmvq_warm()
+    for n in (1, 2, 4, 8):
+        bits = []
+        for dw in bases:
+            y, s = empty((n, rows), torch.float32), empty((n, rows, K // 32), torch.int32)
+            q4mi.check(gpu.q4mi_mmvq(ty, P(dw), rows, K, P(dq), P(dd), n, P(y), 1.0, P(s)),
+                       "q4mi_mmvq")
+            y2 = empty((n, rows), torch.float32)
+            q4mi.check(gpu.q4_mmvq_n(ty, P(dw), rows, K, P(dx), P(y2), 1.0, n), "q4_mmvq_n")
+            assert np.array_equal(host(y).view(np.uint32), host(y2).view(np.uint32))
+            bits.append(host(y).view(np.uint32))
+            sums = host(s)
+            for t in {0, n - 1}:
+                for r in {0, rows // 2, rows - 1}:
+                    want = oracle.group_sums(ty, w[r * rb:(r + 1) * rb], K, q[t])
+                    assert np.array_equal(sums[t, r], want), (t, r)
+        assert np.array_equal(bits[0], bits[1]), n
+        if n in (1, 8):
+            m = min(rows, 200)
+            assert rel_err(host(y)[:, :m], oracle.dot8_rows(ty, w[:m * rb], m, K, x[:n])) <= 1e-3
+
+
+@pytest.mark.parametrize("ty", GEMV_TYPES)
+@pytest.mark.parametrize("K", [4096, 8192])
+def test_gemv_lane_layouts_same_bits(gpu, ty, K):
+    """Rows of 128 and 256 groups: the 64-lane layout (one token, or few rows)
+    and the 32-lane one (many rows, three tokens and more) give the same bits."""
+    import torch
+    rows = 32768 + 5
+    bv, bs, at = {T_IQ3_S: (256, 110, 0), T_Q8_0: (32, 34, 0), T_IQ4_NL: (32, 18, 0),
+                  T_Q2_0: (64, 18, 0), T_IQ2_S: (256, 82, 0), T_Q6_K: (256, 210, 208)}[ty]
+    gen = torch.Generator("cuda").manual_seed(ty + K)
+    w = torch.randint(0, 256, (rows * K // bv, bs), dtype=torch.uint8, device="cuda", generator=gen)
+    w[:, at + 1] = w[:, at + 1] % 8 + 0x10          # block scales 2^-11 .. 2^-9
+    x = torch.randn((5, K), device="cuda", generator=gen)
+    few = 300 * (K // bv) * bs
+    ys = []
+    for n, r in ((1, rows), (3, rows), (5, rows), (5, 300)):
+        y = torch.empty((n, r), device="cuda")
+        ww = w if r == rows else w.view(-1)[:few]
+        q4mi.check(gpu.q4_mmvq_n(ty, q4mi.ptr(ww), r, K, q4mi.ptr(x), q4mi.ptr(y), 1.0, n),
+                   "q4_mmvq_n")
+        ys.append(y)
+    one, three, five, short = ys
+    assert bool(torch.isfinite(five).all())
+    assert torch.equal(one[0], three[0]) and torch.equal(three, five[:3])
+    assert torch.equal(five[:, :300], short)
