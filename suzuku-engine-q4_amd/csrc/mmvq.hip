@@ -332,8 +332,9 @@ static bool unit_launch(const uint8_t *W, uint32_t rows, const float *xf, const 
     const size_t lds = Unit<TY>::kTabBytes + (size_t)NT * K + (size_t)NT * (K / 32) * 4;
     // one block per CU (each task at least one row set); the types without
     // tables to build take up to four times as many for a tall matrix, which
-    // the CUs then share by their actual rate (Q8_0 151936 x 2048, 1 / 4
-    // tokens: 62.2 / 65.8 us with one block per CU, 57.8 / 64.5 with four)
+    // the CUs then share by their actual rate (151936 x 2048, 1 / 4 tokens,
+    // one block per CU and four: Q8_0 64.1 / 67.2 and 60.0 / 66.1 us, IQ4_NL
+    // 36.8 / 51.1 and 34.9 / 45.4, Q2_0 26.3 / 42.3 and 22.9 / 35.5)
     const uint32_t tasks = (rows + RPW - 1) / RPW, cus = (uint32_t)cu_count();
     const uint32_t most = Unit<TY>::kTabBytes ? 1u : 4u;
     const uint32_t grid = std::min(cus * std::max(1u, std::min(most, tasks / (64u * cus))), tasks);
@@ -402,15 +403,22 @@ static bool unit_any(const uint8_t *W, uint32_t rows, uint32_t K, const float *x
 // columns, 1-8 tokens: 0.67 of the tile kernel's time in the geometric mean)
 // but for the tall Q8_0 matrices at one or two tokens, where the tile
 // kernel's many short blocks stream closer to the memory's rate.  Tile /
-// register kernel, us: 151936 x 2048 37.8 / 40.6 (1 token), 39.5 / 40.5 (2),
-// 49.7 / 44.2 (4); 70000 x 2048 19.5 / 19.7 and 20.8 / 20.3 (1, 2);
-// 151936 x 4096 83.4 / 80.8 (2).  The two give a row the same bits where
-// both take part (Q8_0), so a row's result still does not depend on nt.
+// register kernel, us, over 0.7-1.5 GB of distinct matrices (runs differ by 1 to 2 %):
+//   1 token, columns      1024          2048          4096          8192
+//     112 MB          23.1 / 23.7   22.7 / 22.7   23.3 / 21.6   23.6 / 22.6
+//     144 MB          27.8 / 29.0   27.5 / 27.5   27.9 / 27.3   28.7 / 27.7
+//     208 MB          38.4 / 42.0   37.4 / 39.8   38.1 / 39.2   38.5 / 39.0
+//     331 MB          58.1 / 63.2   58.1 / 61.5   58.3 / 59.0   57.8 / 60.6
+//   2 tokens
+//     144 MB          28.8 / 29.5   29.0 / 28.3   31.0 / 28.8   32.0 / 28.5
+//     208 MB          39.8 / 42.4   39.5 / 41.0   42.1 / 41.3   42.9 / 40.3
+//     331 MB          61.2 / 64.1   60.4 / 61.3   63.4 / 62.0   63.9 / 62.0
+//     500 MB          89.0 / 97.0   87.7 / 91.7   92.8 / 90.4   92.1 / 91.1
 static bool unit_ok(uint32_t ty, const uint8_t *W, uint64_t rows, uint64_t K, uint32_t nt) {
     const uint64_t rb = q4mi_row_bytes(ty, K), bytes = rows * rb;
     if (((uintptr_t)W & 3u) || rb % 4) return false;
     if (ty != Q4MI_T_Q8_0 || nt > 2) return true;
-    return nt == 1 ? bytes < (144ull << 20) : bytes < (160ull << 20) || K > 2560;
+    return bytes < (160ull << 20) || (nt == 2 && K > 2560);
 }
 
 // weight bytes per row tile
@@ -553,9 +561,9 @@ bool mmvq_q8(uint32_t ty, const uint8_t *W, uint64_t rows, uint64_t K, const int
 // Activations quantized inside the tile kernel's blocks: used while the codes
 // of the padded token count fit 16 KB of LDS beside the tile and the call has at
 // most 1024 row tiles.  Every block re-reads and re-quantizes all of x, so
-// a tall matrix (config 4: 18992 tiles) is faster with one quantize launch
-// (measured: 56.5 against 70.8 us at 1 token), a short one (config 0: 512
-// tiles) without it (7.97 against 7.32 us).
+// a tall matrix (Q8_0 151936 x 2048: 18992 tiles) is faster with one quantize
+// launch (measured: 56.5 against 70.8 us at 1 token), a short one (IQ3_S 4096 x
+// 4096: 512 tiles) without it (7.97 against 7.32 us).
 static bool mmvq_fused_fits(uint32_t ty, uint64_t rows, uint64_t K, uint32_t nt) {
     const uint32_t ntp = nt == 1 ? 1 : nt == 2 ? 2 : nt <= 4 ? 4 : 8;
     if ((uint64_t)ntp * K > 16384) return false;
@@ -608,8 +616,9 @@ void q4_mmvq_release(void) {
 }
 
 /* y[t*nrows + r] = scale * dot(W row r, q8(x[t])), t < n (1..8).  Types:
- * IQ3_S, Q8_0; ncols a multiple of 256 (IQ3_S) / 32 (Q8_0) with
- * ncols/32 in {8,16,32,64,128,256}.  false = not covered; nothing launched. */
+ * IQ3_S, Q8_0, IQ4_NL, Q2_0, IQ2_S, Q6_K; ncols a whole number of blocks with
+ * ncols/32 in {8,16,20,32,64,80,128,256}.  false = not covered; nothing
+ * launched. */
 bool q4_mmvq_n(uint32_t ty, const uint8_t *d_w, uint64_t nrows, uint64_t ncols,
                const float *d_x, float *d_y, float scale, uint32_t n) {
     if (!q4_mmvq_on() || n < 1 || n > 8 || !d_w || !d_x || !d_y || !nrows ||
