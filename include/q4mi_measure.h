@@ -17,7 +17,9 @@ extern "C" {
 #endif
 
 /* Which launches of the decode pair run: 1 = gate/up only, 2 = down only,
- * 3 = both (default).  Lets a benchmark time each kernel alone. */
+ * 3 = both (default).  Lets a benchmark time each kernel alone: a down launch
+ * by itself takes the call's own lists and the h rows left by the last gate/up
+ * launch (over device lists a small launch ahead of it lays out the plan). */
 void q4mi_moe_phases(int mask);
 /* Accepted and without effect: the decode kernels hold their weights in
  * registers and have no LDS ring to shorten. */

@@ -5,9 +5,33 @@
 namespace q4mi {
 
 // Measurement hook: bit 0 runs the gate/up launch, bit 1 the down launch
-// (default both).  Lets a benchmark time each kernel of the pair alone (a
-// down launch over device lists reads the last gate/up launch's plan).
+// (default both).  Lets a benchmark time each kernel of the pair alone.
 static int g_phases = 3;
+
+#ifdef Q4MI_MEASURE
+// The plan of a down launch over device lists that no gate/up launch of the
+// same call precedes (with one, its block 0 publishes the plan).
+template <bool LG>
+__global__ __launch_bounds__(64) void plan_k(Plan *g, ListSrc s) {
+    __shared__ Plan P;
+    __shared__ uint32_t ht[kPlanTable / 4];
+    const uint32_t lane = threadIdx.x;
+    const PlanLane l = build_plan<LG>(&P, s, lane, ht);
+    __syncthreads();
+    finish_plan(&P, l, lane);
+    __syncthreads();
+    for (uint32_t i = lane; i < sizeof(Plan) / 16; i += 64) ((uint4 *)g)[i] = ((const uint4 *)&P)[i];
+}
+
+static bool down_alone_plan(const MoeArgs &a) {
+    if ((g_phases & 1) || a.src.unique) return true;
+    if (a.src.lg) plan_k<true><<<dim3(1), dim3(64), 0, stream()>>>(a.gplan, a.src);
+    else plan_k<false><<<dim3(1), dim3(64), 0, stream()>>>(a.gplan, a.src);
+    return launch_ok("plan_k");
+}
+#else
+static bool down_alone_plan(const MoeArgs &) { return true; }
+#endif
 
 template <int NT>
 static bool run_nt(uint32_t ty_gu, uint32_t ty_dn, const MoeArgs &a, uint32_t nu_host) {
@@ -18,6 +42,7 @@ static bool run_nt(uint32_t ty_gu, uint32_t ty_dn, const MoeArgs &a, uint32_t nu
         if (!ok) return false;
     }
     if (!(g_phases & 2)) return true;
+    if (!down_alone_plan(a)) return false;
     return ty_dn == Q4MI_T_IQ3_S ? dn_dispatch<Q4MI_T_IQ3_S, NT>(a, nu_host)
          : ty_dn == Q4MI_T_Q8_0  ? dn_dispatch<Q4MI_T_Q8_0, NT>(a, nu_host)
                                  : moe_fmt_dn(ty_dn, NT, a, nu_host);

@@ -323,6 +323,42 @@ def test_ring_reuse_matches(gpu_meas, oracle):
         gpu_meas.q4mi_moe_lds_cap(0)
 
 
+def test_down_launch_alone_takes_the_calls_lists(gpu_meas, oracle):
+    """The measurement build's down launch by itself, over device lists (one
+    token, and a 4-token window): the h rows of the last gate/up launch, the
+    expert list and weights of its own call.  So with the same experts and
+    other weights it gives the full layer's y at those weights bit for bit."""
+    ly = layer()
+    rng = np.random.default_rng(25)
+    for n_tok in (1, 4):
+        x = dev(rng.standard_normal((n_tok, ly.n_embd)).astype(np.float32))
+        es = np.full((n_tok, 64), -1, np.int32)
+        for t in range(n_tok):
+            es[t, :8] = rng.choice(512, 8, replace=False)
+        d_es, d_n = dev(es), dev(np.full(n_tok, 8, np.int32))
+
+        def run(ew, phases):
+            y = dev(np.zeros((n_tok, ly.n_embd), np.float32))
+            gpu_meas.q4mi_moe_phases(phases)
+            try:
+                lists = (q4mi.ptr(ly.d_arena), ly.stride, q4mi.ptr(d_es), q4mi.ptr(ew), q4mi.ptr(d_n))
+                packed = (T_IQ3_S, ly.og, T_IQ3_S, ly.ou, T_IQ3_S, ly.od, q4mi.ptr(x))
+                out = (q4mi.ptr(y), ly.n_ff, ly.n_embd, ly.n_embd)
+                if n_tok == 1:
+                    ok = gpu_meas.q4_hip_moe_exec_dev(*lists, *packed, None, None, None, *out)
+                else:
+                    ok = gpu_meas.q4_hip_moe_exec_win(*lists, n_tok, *packed, None, *out)
+                q4mi.check(ok, "down launch", gpu_meas)
+            finally:
+                gpu_meas.q4mi_moe_phases(3)
+            return host(y).view(np.uint32)
+
+        wa, wb = (dev(rng.random((n_tok, 64)).astype(np.float32)) for _ in range(2))
+        want = run(wb, 3)
+        run(wa, 3)
+        assert np.array_equal(run(wb, 2), want), n_tok
+
+
 def test_moe_exec_dev_and_rejects(gpu, oracle):
     import torch
     ly = layer()
