@@ -50,6 +50,10 @@ uint64_t q4mi_alloc_count(void);
  * buffer is retired, not freed) run on host fakes without a device; 1 =
  * every case behaves as documented. */
 int q4mi_grow_selftest(void);
+/* The once-a-device marks of kernel attributes (a second device of the process
+ * sets them again; a failure is tried again), on the host alone; 1 = every
+ * case behaves as documented. */
+int q4mi_per_device_selftest(void);
 
 #ifdef __cplusplus
 }

@@ -317,19 +317,9 @@ static bool unit_launch(const uint8_t *W, uint32_t rows, const float *xf, const 
                         const float *xd, uint32_t nt, float *y, float scale, int32_t *sums) {
     constexpr uint32_t K = 64 * LPR * UPL, RPW = 64 / LPR;
     const auto kern = mmvq_u_k<TY, NT, LPR, UPL, XF>;
-    static bool ready = false;
-    if (!ready) {
-        // the table lookups take the dynamic LDS to start at offset 0
-        hipFuncAttributes fa;
-        if (hipFuncGetAttributes(&fa, (const void *)kern) != hipSuccess || fa.sharedSizeBytes != 0 ||
-            hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024) != hipSuccess) {
-            set_error("mmvq: LDS limit");
-            return false;
-        }
-        ready = true;
-    }
     const size_t lds = Unit<TY>::kTabBytes + (size_t)NT * K + (size_t)NT * (K / 32) * 4;
+    static DynLds state;
+    if (!dyn_lds_ok((const void *)kern, lds, 160 * 1024, state, "mmvq_u_k")) return false;
     // one block per CU (each task at least one row set); the types without
     // tables to build take up to four times as many for a tall matrix, which
     // the CUs then share by their actual rate (151936 x 2048, 1 / 4 tokens,

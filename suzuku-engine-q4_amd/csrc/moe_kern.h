@@ -751,26 +751,9 @@ __global__ __launch_bounds__(kT) void moe_dn_k(MoeArgs a) {
 constexpr size_t kLdsCap = 160 * 1024;
 
 template <class Kern>
-static bool moe_launch(Kern kern, const MoeArgs &a, uint32_t grid, size_t lds, bool &ready,
+static bool moe_launch(Kern kern, const MoeArgs &a, uint32_t grid, size_t lds, DynLds &st,
                        const char *name) {
-    if (lds > kLdsCap) {
-        set_error("%s: LDS limit", name);
-        return false;
-    }
-    if (!ready) {
-        // the table lookups take the dynamic LDS to start at offset 0
-        hipFuncAttributes fa;
-        if (hipFuncGetAttributes(&fa, (const void *)kern) != hipSuccess || fa.sharedSizeBytes != 0) {
-            set_error("%s: unexpected static LDS", name);
-            return false;
-        }
-        if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)kLdsCap) != hipSuccess) {
-            set_error("%s: LDS limit (%zu)", name, lds);
-            return false;
-        }
-        ready = true;
-    }
+    if (!dyn_lds_ok((const void *)kern, lds, kLdsCap, st, name)) return false;
     kern<<<dim3(grid), dim3(kT), lds, stream()>>>(a);
     return launch_ok(name);
 }
@@ -782,21 +765,21 @@ constexpr size_t kPlanTable = 4096 + 512;
 template <uint32_t TY, int NT, int LPR, int UPL, int SRC>
 static bool launch_gu(const MoeArgs &a) {
     constexpr uint32_t RPW = 64 / LPR;
-    static bool ready = false;
+    static DynLds state;
     MoeArgs b = a;
     b.tpe = a.n_ff / RPW;
     b.tpe_inv = (uint32_t)((0x100000000ull + b.tpe - 1) / b.tpe);
     const size_t fixed = al16(Unit<TY>::kTabBytes + sizeof(Plan) + (size_t)NT * a.K +
                               (size_t)NT * (a.K / 32) * 8);
     const size_t lds = fixed + std::max(sizeof(GuOut<NT, RPW>) * kW, kPlanTable);
-    return moe_launch(moe_gu_k<TY, NT, LPR, UPL, SRC>, b, (uint32_t)cu_count(), lds, ready,
+    return moe_launch(moe_gu_k<TY, NT, LPR, UPL, SRC>, b, (uint32_t)cu_count(), lds, state,
                       "moe_gu_k");
 }
 
 template <uint32_t TY, int NT, int UPR, int SRC>
 static bool launch_dn(const MoeArgs &a, uint32_t nu_host) {
     constexpr uint32_t RPW = 64 / UPR, NV = (UPR & (UPR - 1)) == 0 ? 1u : (uint32_t)UPR;
-    static bool ready = false;
+    static DynLds state;
     MoeArgs b = a;
     // rows per block: one block per CU, but no fewer rows than a wave holds
     // (up to 8)
@@ -806,7 +789,7 @@ static bool launch_dn(const MoeArgs &a, uint32_t nu_host) {
     const size_t hb = (size_t)b.nsel_cap * a.n_ff + (size_t)b.nsel_cap * (a.n_ff / 32) * 4;
     const size_t lds = Unit<TY>::kTabBytes + hb + (size_t)kW * NT * RPW * NV * 4;
     return moe_launch(moe_dn_k<TY, NT, UPR, SRC>, b, (a.n_embd + b.dn_rows - 1) / b.dn_rows, lds,
-                      ready, "moe_dn_k");
+                      state, "moe_dn_k");
 }
 
 template <uint32_t TY, int NT, int LPR, int UPL>

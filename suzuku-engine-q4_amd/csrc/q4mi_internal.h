@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <atomic>
 #include <vector>
 
 #include "../../include/q4mi.h"
@@ -92,6 +93,56 @@ inline bool launch_ok(const char *what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("%s: launch failed: %s", what, hipGetErrorString(e));
+        return false;
+    }
+    return true;
+}
+
+// Work done once on each device a process uses (kernel attributes belong to
+// the current device): run(dev, f) calls f unless it has succeeded for dev.
+// Two threads may both call f the first time, so f must be repeatable.
+class PerDevice {
+    std::atomic<uint64_t> done_{0};
+
+public:
+    template <class F>
+    bool run(int dev, F f) {
+        const uint64_t bit = dev >= 0 && dev < 64 ? 1ull << dev : 0;
+        if (done_.load(std::memory_order_acquire) & bit) return true;
+        if (!f()) return false;
+        done_.fetch_or(bit, std::memory_order_release);
+        return true;
+    }
+};
+
+// Launch state of a kernel that takes its dynamic LDS at offset 0.
+struct DynLds {
+    std::atomic<bool> checked{false};
+    PerDevice limit;
+};
+// Before a launch with `lds` bytes of dynamic LDS, at most `cap`: the kernel
+// has no static LDS, and more than the default 64 KB is allowed on the current
+// device (a launch within them needs no device query).
+inline bool dyn_lds_ok(const void *kern, size_t lds, size_t cap, DynLds &st, const char *name) {
+    if (lds > cap) {
+        set_error("%s: LDS limit (%zu)", name, lds);
+        return false;
+    }
+    if (!st.checked.load(std::memory_order_acquire)) {
+        hipFuncAttributes fa;
+        if (hipFuncGetAttributes(&fa, kern) != hipSuccess || fa.sharedSizeBytes != 0) {
+            set_error("%s: unexpected static LDS", name);
+            return false;
+        }
+        st.checked.store(true, std::memory_order_release);
+    }
+    if (lds <= 65536) return true;
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || !st.limit.run(dev, [&] {
+            return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)cap) ==
+                   hipSuccess;
+        })) {
+        set_error("%s: LDS limit (%zu)", name, lds);
         return false;
     }
     return true;

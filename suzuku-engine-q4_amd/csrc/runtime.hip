@@ -129,6 +129,23 @@ int q4mi_grow_selftest(void) {
         return 0;
     return 1;
 }
+
+int q4mi_per_device_selftest(void) {
+    q4mi::PerDevice p;
+    int calls = 0;
+    bool fail = true;
+    auto f = [&] {
+        calls++;
+        return !fail;
+    };
+    if (p.run(0, f) || p.run(0, f) || calls != 2) return 0;   // a failure is tried again
+    fail = false;
+    if (!p.run(0, f) || !p.run(0, f) || calls != 3) return 0;   // once a device
+    if (!p.run(7, f) || !p.run(63, f) || calls != 5) return 0;   // and once on each
+    if (!p.run(0, f) || !p.run(7, f) || !p.run(63, f) || calls != 5) return 0;
+    if (!p.run(64, f) || !p.run(64, f) || calls != 7) return 0;   // past the marks: each time
+    return 1;
+}
 #endif
 
 const char *q4mi_status_text(uint32_t bits) {

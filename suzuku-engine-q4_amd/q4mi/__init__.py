@@ -126,6 +126,7 @@ _MEAS_SIGS = {
     "q4mi_mmq_ab_probe": (_c.c_bool, [_c.c_int, _u32, _c.POINTER(_c.c_uint64)]),
     "q4mi_alloc_count": (_c.c_uint64, []),
     "q4mi_grow_selftest": (_c.c_int, []),
+    "q4mi_per_device_selftest": (_c.c_int, []),
 }
 
 _lib = None

@@ -139,6 +139,13 @@ def test_grow_policy_selftest():
     assert M.q4mi_grow_selftest() == 1
 
 
+def test_kernel_attributes_once_a_device():
+    """The LDS limit of a decode or GEMV kernel is raised once on each device
+    that launches it, not once a process."""
+    M = q4mi.meas()
+    assert M.q4mi_per_device_selftest() == 1
+
+
 def test_status_text_xg_tiles():
     L = q4mi.lib()
     t = L.q4mi_status_text(4).decode()
