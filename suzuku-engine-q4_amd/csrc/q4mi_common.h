@@ -99,9 +99,8 @@ __device__ inline uint32_t q4mi_quant_team8(float4 v, float *d, int *bs) {
 // take short forms that give the same bits:
 //   a / 127   one multiply by RN(1/127) and one residual step,
 //   127 / a   the hardware reciprocal, one Newton step and one residual step
-//             (both equal the IEEE divide for every mantissa, checked over
-//             all 2^23; away from overflow and underflow the exponent does
-//             not matter),
+//             (both equal the IEEE divide for every mantissa, and at both
+//             ends of the range: test_in_block_quantizer_every_mantissa),
 //   the code  RN(x * sc) + 1.5 * 2^23 leaves the integer, rounded to nearest
 //             even, in the low bits (|x * sc| <= 127 there).
 // Anything else takes q4mi_q8_code and the IEEE divides.

@@ -199,3 +199,55 @@ def test_gemv_lane_layouts_same_bits(gpu, ty, K):
     assert bool(torch.isfinite(five).all())
     assert torch.equal(one[0], three[0]) and torch.equal(three, five[:3])
     assert torch.equal(five[:, :300], short)
+
+
+# exponents of a group's largest magnitude: the short divisions' range is 2^-100 .. 2^100
+# (both ends inside); the rest of the float range takes the full divides
+@pytest.mark.parametrize("exps,calls", [((0,), 4096), ((-100,), 32), ((-101,), 32), ((-126,), 32),
+                                        ((99,), 32), ((100,), 32), ((126,), 32),
+                                        ((-126, -101, -100, -30, 0, 40, 99, 100, 126), 64)])
+def test_in_block_quantizer_every_mantissa(gpu, exps, calls):
+    """The quantizer inside the decode, window and GEMV kernels (eight values a
+    lane, short exact divisions) gives the scales and codes of q4mi_quant8's
+    IEEE divides bit for bit: all 2^23 mantissas of a group's largest magnitude
+    at exponent 0, 65536 evenly spread ones (first and last among them) at the
+    ends of the short range and beyond, and exponents mixed within a wave.  The
+    other values are the 126.5 .. 0.5 steps, where the code rounds to even, and
+    their neighbours.  An identity matrix (Q8_0, block scales 1) shows every
+    value's code times its group's scale, one rounding of the two."""
+    import torch
+    K, n = 8192, 8
+    dv = dict(device="cuda")
+    w = torch.zeros((K, K // 32, 34), dtype=torch.uint8, **dv)
+    w[:, :, 1] = 0x3c                                        # fp16 1.0
+    r = torch.arange(K, **dv)
+    w[r, r // 32, 2 + r % 32] = 1
+    gen = torch.Generator("cuda").manual_seed(calls)
+    groups = n * K // 32
+    last = (1 << 23) - 1
+    bad = torch.zeros((), dtype=torch.int64, **dv)
+    P = q4mi.ptr
+    for c in range(calls):
+        at = torch.arange(c * groups, (c + 1) * groups, **dv)
+        man = (at * last).div(calls * groups - 1, rounding_mode="floor")
+        e = torch.tensor(exps, **dv)[torch.randint(0, len(exps), (groups,), generator=gen, **dv)]
+        a = (((e + 127) << 23) | man).to(torch.int32).view(torch.float32)[:, None]
+        step = torch.randint(-127, 127, (groups, 32), generator=gen, **dv) + 0.5
+        x = (step / 127 * a)
+        near = torch.randint(-1, 2, (groups, 32), generator=gen, dtype=torch.int32, **dv)
+        x = (x.view(torch.int32) + near).view(torch.float32)
+        pos = torch.randint(0, 32, (groups, 1), generator=gen, **dv)
+        x.scatter_(1, pos, torch.where(pos % 2 == 0, a, -a))
+        x = x.reshape(n, K).contiguous()
+        q = torch.empty((n, K), dtype=torch.int8, **dv)
+        d = torch.empty((n, K // 32), **dv)
+        bs = torch.empty((n, K // 32), dtype=torch.int32, **dv)
+        y = torch.empty((n, K), **dv)
+        q4mi.check(gpu.q4mi_quant8(P(x), None, n, K, P(q), P(d), P(bs)), "q4mi_quant8")
+        q4mi.check(gpu.q4_mmvq_n(T_Q8_0, P(w), K, K, P(x), P(y), 1.0, n), "q4_mmvq_n")
+        want = q.float() * d.repeat_interleave(32, dim=1)
+        bad += (y != want).sum()
+        if c == 0:
+            # (-128: every code of a group at -126, whose 127 / a is infinite)
+            assert int(q.int().abs().max()) >= 127 and bool(torch.isfinite(want).all())
+    assert int(bad) == 0
