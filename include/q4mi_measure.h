@@ -3,8 +3,7 @@
  *
  * The product library (libq4mi.so) does not export these: each changes
  * process-global behaviour (a benchmark that runs only one kernel of the
- * decode pair, a test that shrinks the kernels' LDS), which no production
- * caller may reach.  None has a reference counterpart.
+ * decode pair) or reports internal state, which no production caller needs.  None has a reference counterpart.
  */
 #ifndef Q4MI_MEASURE_H
 #define Q4MI_MEASURE_H
@@ -21,9 +20,6 @@ extern "C" {
  * by itself takes the call's own lists and the h rows left by the last gate/up
  * launch (over device lists a small launch ahead of it lays out the plan). */
 void q4mi_moe_phases(int mask);
-/* Accepted and without effect: the decode kernels hold their weights in
- * registers and have no LDS ring to shorten. */
-void q4mi_moe_lds_cap(uint32_t bytes);
 /* One launch of an MFMA throughput probe on the library stream (kind 0:
  * int8 32x32x32, 1: fp16 32x32x16); *ops = the launch's ops, for a
  * caller-timed rate. */
@@ -32,7 +28,7 @@ bool q4mi_mfma_probe(int kind, uint32_t iters, uint64_t *ops);
  * `waves` producer waves copy per_block bytes (src + block * per_block)
  * into LDS with 1 KB global_load_lds_dwordx4 operations and wait for them;
  * per_block = 0 launches the same grid empty.  *bytes = the launch's
- * total.  The floors of the decode kernels' structure. */
+ * total.  A floor of launches that copy through LDS. */
 bool q4mi_stream_probe(const void *src, uint32_t per_block, uint32_t waves, uint64_t *bytes);
 /* One launch of the plain streaming probe, the chip's own floor: `bytes`
  * (a multiple of 4096 * unroll) read from src by 256-thread blocks with

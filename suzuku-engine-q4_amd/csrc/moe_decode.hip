@@ -48,8 +48,8 @@ static bool run_nt(uint32_t ty_gu, uint32_t ty_dn, const MoeArgs &a, uint32_t nu
                                  : moe_fmt_dn(ty_dn, NT, a, nu_host);
 }
 
-// Rows are staged with 4- or 16-byte copies, so a row's byte size must be a
-// multiple of 4 (IQ3_S, IQ2_S, IQ2_XXS, IQ2_XS, IQ3_XXS: K a multiple of
+// A row's fields are read as the whole dwords around them, so its byte size
+// must be a multiple of 4 (IQ3_S, IQ2_S, IQ2_XXS, IQ2_XS, IQ3_XXS: K a multiple of
 // 512; Q8_0, IQ4_NL, Q2_0: of 64; IQ4_XS: of 256).  Gate/up: IQ3_S, Q8_0,
 // IQ2_S, IQ2_XXS, IQ2_XS, IQ3_XXS, IQ4_XS; down: IQ3_S, Q8_0, IQ2_S, IQ4_NL,
 // Q2_0.
@@ -255,10 +255,6 @@ extern "C" {
 /* Measurement build only (libq4mi_meas.so): 1 = gate/up launch only, 2 =
  * down only, 3 = both. */
 void q4mi_moe_phases(int mask) { g_phases = mask & 3; }
-
-/* Measurement build only: accepted and without effect (the decode kernels
- * hold their weights in registers; there is no LDS ring to shorten). */
-void q4mi_moe_lds_cap(uint32_t bytes) { (void)bytes; }
 #endif
 
 /* Copy the fp32 h of the last decode call, [64 unique experts][8 tokens]

@@ -18,7 +18,7 @@ PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 # Q4MI_LIB selects another build of the same library (same ABI).
 LIB_PATH = os.environ.get("Q4MI_LIB") or os.path.join(PKG, "lib", "libq4mi.so")
 # The measurement build (-DQ4MI_MEASURE): the same ABI plus the hooks of
-# include/q4mi_measure.h.  Benchmarks and LDS-ring tests load it beside the
+# include/q4mi_measure.h.  Benchmarks and tests load it beside the
 # product library; its state (stream, scratch) is its own.
 MEAS_PATH = os.path.join(PKG, "lib", "libq4mi_meas.so")
 
@@ -119,7 +119,6 @@ _SIGS = {
 # measurement build only
 _MEAS_SIGS = {
     "q4mi_moe_phases": (None, [_c.c_int]),
-    "q4mi_moe_lds_cap": (None, [_u32]),
     "q4mi_mfma_probe": (_c.c_bool, [_c.c_int, _u32, _c.POINTER(_c.c_uint64)]),
     "q4mi_stream_probe": (_c.c_bool, [_vp, _u32, _u32, _c.POINTER(_c.c_uint64)]),
     "q4mi_plain_stream_probe": (_c.c_bool, [_vp, _c.c_uint64, _u32]),

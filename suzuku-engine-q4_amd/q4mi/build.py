@@ -3,8 +3,8 @@
 Every source under csrc/ is compiled by hipcc for gfx950 only and linked
 into one shared object exposing the C ABI declared in include/q4mi.h.  The
 same sources compiled with -DQ4MI_MEASURE give lib/libq4mi_meas.so, which
-adds the measurement hooks of include/q4mi_measure.h (benchmarks and the
-LDS-ring tests load it; the product library never exports them).
+adds the measurement hooks of include/q4mi_measure.h (benchmarks and tests
+load it; the product library never exports them).
 """
 import concurrent.futures as cf
 import glob

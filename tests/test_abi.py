@@ -105,8 +105,8 @@ def _exports(path):
 
 def test_measurement_hooks_only_in_measurement_build():
     """The hooks that change process-global behaviour (run one kernel of the
-    decode pair, shrink the decode LDS, the MFMA probe) are exported by the
-    measurement build only; it also carries the whole product ABI."""
+    decode pair, the probes) are exported by the measurement build only; it
+    also carries the whole product ABI."""
     text = re.sub(r"/\*.*?\*/", "", open(MEAS_HEADER).read(), flags=re.S)
     hooks = sorted(set(re.findall(r"\b(q4mi_\w+)\s*\(", text)))
     assert hooks == sorted(q4mi.measurement_symbols())

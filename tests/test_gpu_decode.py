@@ -265,62 +265,43 @@ def test_moe_decode_config2(gpu, oracle):
     assert np.array_equal(y.view(np.uint32), y3.view(np.uint32))
 
 
-def test_ring_reuse_matches(gpu_meas, oracle):
-    """Decode kernels whose LDS ring is smaller than their share (chunks reuse
-    slots; 3 slots for 4 producers, where a slot's successive chunks belong
-    to different producers) give the unconstrained run's y bit for bit:
-    host list, device list (8 experts) and a 4-token window.  (Without the
-    ring's per-slot owner check the down kernel returned wrong rows here.)"""
-    import torch
+def test_list_sources_same_bits(gpu, oracle):
+    """A token's y does not depend on where its expert list comes from or on the
+    tokens beside it: a host list, a device list, and 2-, 4- and 8-token windows
+    whose tokens all picked the same experts (8 and 64 / n_tok of them) give the
+    same bits (each is an instantiation of its own, with its own shares of the
+    rows), and the host list's y is the oracle's to 1e-3."""
     ly = layer()
     rng = np.random.default_rng(24)
-    x = rng.standard_normal(ly.n_embd).astype(np.float32)
-    ids, wts = routed_ids(oracle, rng)
-    ids = np.append(ids, 512).astype(np.int32)
-    wts = np.append(wts, 1.0).astype(np.float32)
-    es = np.full(64, -1, np.int32)
-    ew = np.zeros(64, np.float32)
-    es[:8], ew[:8] = ids[:8], wts[:8]
-    d_es, d_ew, d_n, dx = dev(es), dev(ew), dev(np.array([8], np.int32)), dev(x)
-    xw = rng.standard_normal((4, ly.n_embd)).astype(np.float32)
-    lgw = rng.standard_normal((4, 512)).astype(np.float32)
-    wid, wwt = oracle.softmax_topk(lgw, 10)
-    wes = np.full((4, 64), -1, np.int32)
-    wew = np.zeros((4, 64), np.float32)
-    wes[:, :10], wew[:, :10] = wid, wwt
-    d_wid, d_wwt, d_wn, dxw = dev(wes), dev(wew), dev(np.full(4, 10, np.int32)), dev(xw)
-
-    def run(window=True, devlist=True):
-        y_host = moe_exec_host(gpu_meas, ly, x, ids, wts)
-        if not devlist:
-            return [y_host]
+    x = rng.standard_normal((8, ly.n_embd)).astype(np.float32)
+    packed = (T_IQ3_S, ly.og, T_IQ3_S, ly.ou, T_IQ3_S, ly.od)
+    size = (ly.n_ff, ly.n_embd, ly.n_embd)
+    P = q4mi.ptr
+    ids_all, wts_all = routed_ids(oracle, rng, k=32)
+    for k in (8, 16, 32):
+        ids, wts = ids_all[:k], wts_all[:k]
+        y = [moe_exec_host(gpu, ly, x[t], ids, wts).view(np.uint32) for t in range(8)]
+        yo = oracle.moe_tokens(ly.n_embd, ly.n_ff, T_IQ3_S, T_IQ3_S, ly.arena, ly.stride, x[:1],
+                               ids[None], wts[None])[0]
+        assert rel_err(y[0].view(np.float32), yo) <= TOL
+        es = np.full((8, 64), -1, np.int32)
+        ew = np.zeros((8, 64), np.float32)
+        es[:, :k], ew[:, :k] = ids, wts
+        d_es, d_ew, d_n, dx = dev(es), dev(ew), dev(np.full(8, k, np.int32)), dev(x)
         yd = dev(np.zeros(ly.n_embd, np.float32))
-        q4mi.check(gpu_meas.q4_hip_moe_exec_dev(q4mi.ptr(ly.d_arena), ly.stride, q4mi.ptr(d_es),
-                                           q4mi.ptr(d_ew), q4mi.ptr(d_n), T_IQ3_S, ly.og,
-                                           T_IQ3_S, ly.ou, T_IQ3_S, ly.od, q4mi.ptr(dx), None,
-                                           None, None, q4mi.ptr(yd), ly.n_ff, ly.n_embd,
-                                           ly.n_embd), "exec_dev")
-        if not window:
-            return [y_host, host(yd)]
-        yw = dev(np.zeros((4, ly.n_embd), np.float32))
-        q4mi.check(gpu_meas.q4_hip_moe_exec_win(q4mi.ptr(ly.d_arena), ly.stride, q4mi.ptr(d_wid),
-                                           q4mi.ptr(d_wwt), q4mi.ptr(d_wn), 4, T_IQ3_S, ly.og,
-                                           T_IQ3_S, ly.ou, T_IQ3_S, ly.od, q4mi.ptr(dxw), None,
-                                           q4mi.ptr(yw), ly.n_ff, ly.n_embd, ly.n_embd),
-                   "exec_win")
-        return [y_host, host(yd), host(yw)]
-
-    base = run()
-    try:
-        # 120 KB: the window's rings reuse slots (down 2 slots, gate/up 5);
-        # 80 KB: the device list's down ring does (3 slots, 8 chunks);
-        # 70 / 59 KB: the host list's gate/up ring does (3 or 4 slots)
-        for cap in (120000, 81920, 72000, 60000):
-            gpu_meas.q4mi_moe_lds_cap(cap)
-            for got, want in zip(run(window=cap >= 120000, devlist=cap >= 81920), base):
-                assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), cap
-    finally:
-        gpu_meas.q4mi_moe_lds_cap(0)
+        q4mi.check(gpu.q4_hip_moe_exec_dev(P(ly.d_arena), ly.stride, P(d_es), P(d_ew), P(d_n),
+                                           *packed, P(dx), None, None, None, P(yd), *size),
+                   "exec_dev")
+        assert np.array_equal(host(yd).view(np.uint32), y[0]), k
+        for n in (2, 4, 8):
+            if n * k > 64:
+                continue
+            yw = dev(np.zeros((n, ly.n_embd), np.float32))
+            q4mi.check(gpu.q4_hip_moe_exec_win(P(ly.d_arena), ly.stride, P(d_es), P(d_ew), P(d_n),
+                                               n, *packed, P(dx), None, P(yw), *size), "exec_win")
+            got = host(yw).view(np.uint32)
+            for t in range(n):
+                assert np.array_equal(got[t], y[t]), (k, n, t)
 
 
 def test_down_launch_alone_takes_the_calls_lists(gpu_meas, oracle):
