@@ -263,52 +263,10 @@ struct MoeArgs {
 };
 
 // The kernel's own argument block (kernel parameters start at offset 0 of
-// the kernarg segment).  Uniform reads through it are scalar loads, and the
-// host list can be copied from it into LDS like any other global bytes.
+// the kernarg segment).  Uniform reads through it are scalar loads: a host
+// list's ids and weights are read where they are used.
 typedef const __attribute__((address_space(4))) MoeArgs *KArgs;
 __device__ inline KArgs kargs() { return (KArgs)__builtin_amdgcn_kernarg_segment_ptr(); }
-
-// The host list's ids, one per lane (lane u holds id u), gathered with
-// constant-offset scalar loads (a vector load of the kernel arguments costs
-// a full memory round trip at kernel start).
-typedef const __attribute__((address_space(4))) int32_t *KWords;
-
-template <int K>
-__device__ inline int32_t put_lane(int32_t v, int32_t s) {
-    asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(s), "i"(K));
-    return v;
-}
-// Words [16B, 16B + 16) of w into lanes 16B.. of v: sixteen constant-offset
-// scalar loads (merged into wide loads) and sixteen v_writelane.
-template <int B>
-__device__ inline int32_t put16(int32_t v, KWords w) {
-    int32_t s[16];
-#pragma unroll
-    for (int k = 0; k < 16; k++) s[k] = w[16 * B + k];
-    v = put_lane<16 * B + 0>(v, s[0]);   v = put_lane<16 * B + 1>(v, s[1]);
-    v = put_lane<16 * B + 2>(v, s[2]);   v = put_lane<16 * B + 3>(v, s[3]);
-    v = put_lane<16 * B + 4>(v, s[4]);   v = put_lane<16 * B + 5>(v, s[5]);
-    v = put_lane<16 * B + 6>(v, s[6]);   v = put_lane<16 * B + 7>(v, s[7]);
-    v = put_lane<16 * B + 8>(v, s[8]);   v = put_lane<16 * B + 9>(v, s[9]);
-    v = put_lane<16 * B + 10>(v, s[10]); v = put_lane<16 * B + 11>(v, s[11]);
-    v = put_lane<16 * B + 12>(v, s[12]); v = put_lane<16 * B + 13>(v, s[13]);
-    v = put_lane<16 * B + 14>(v, s[14]); v = put_lane<16 * B + 15>(v, s[15]);
-    return v;
-}
-// The first n words of w, word k in lane k (entries beyond n keep `fill`).
-__device__ inline int32_t host_words(KWords w, uint32_t n, int32_t fill) {
-    int32_t v = fill;
-    v = put16<0>(v, w);
-    if (n > 16) v = put16<1>(v, w);
-    if (n > 32) v = put16<2>(v, w);
-    if (n > 48) v = put16<3>(v, w);
-    return v;
-}
-__device__ inline int32_t host_ids(KArgs ka, uint32_t n) { return host_words(ka->hl.id, n, -1); }
-__device__ inline float host_weights(KArgs ka, uint32_t n) {
-    return __builtin_bit_cast(float, host_words((KWords)ka->hl.w, n, 0));
-}
-
 
 __host__ __device__ inline size_t al16(size_t v) { return (v + 15) & ~(size_t)15; }
 

@@ -98,7 +98,6 @@ struct Unit<Q4MI_T_IQ3_S> {
     static constexpr uint32_t kTabBytes = 32768;
     static constexpr bool kTwo = false;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 9;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, sg, qh, sc, d, s, hs, ss; };
     struct Raw { Win5 qs; u32x3_t sg; uint32_t qh, sc, d; };
@@ -180,7 +179,6 @@ struct Unit<Q4MI_T_Q8_0> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
     static constexpr bool kOneD = false;
-    static constexpr int kRegs = 17;
     static constexpr bool kRawW = true;
     struct Offs { uint32_t b; };
     struct Raw { u32x4_t q[4]; uint32_t e; };   // 68 bytes: d | qs[32] | d | qs[32]
@@ -215,7 +213,6 @@ struct Unit<Q4MI_T_IQ4_NL> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
     static constexpr bool kOneD = false;
-    static constexpr int kRegs = 9;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t b; };
     struct Raw { u32x4_t q[2]; uint32_t e; };   // 36 bytes: d | qs[16] | d | qs[16]
@@ -252,7 +249,6 @@ struct Unit<Q4MI_T_Q2_0> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 5;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t b, s; };
     struct Raw { Win5 w; };                     // 18 bytes: d | qs[16]
@@ -285,7 +281,6 @@ struct Unit<Q4MI_T_IQ2_S> {
     static constexpr uint32_t kTabBytes = sizeof(Iq2sLds);
     static constexpr bool kTwo = true;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 7;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, sg, qh, sc, d, s, hs, ss; };
     struct Raw { u32x3_t qs, sg; uint32_t qh, sc, d; };
@@ -335,7 +330,6 @@ struct Unit<Q4MI_T_IQ2_XXS> {
     static constexpr uint32_t kTabBytes = sizeof(Iq2xLds<256>);
     static constexpr bool kTwo = false;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 5;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, d, s; };
     struct Raw { Win5 q; uint32_t d; };         // grid bytes | aux, twice
@@ -379,7 +373,6 @@ struct Unit<Q4MI_T_IQ2_XS> {
     static constexpr uint32_t kTabBytes = sizeof(Iq2xLds<512>);
     static constexpr bool kTwo = true;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 6;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, sc, d, s, ss; };
     struct Raw { Win5 q; uint32_t sc, d; };     // 16-bit grid index | sign index << 9
@@ -422,7 +415,6 @@ struct Unit<Q4MI_T_IQ3_XXS> {
     static constexpr uint32_t kTabBytes = sizeof(Iq3xxsLds);
     static constexpr bool kTwo = false;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 7;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, ax, d, s; };
     struct Raw { Win5 q; u32x3_t ax; uint32_t d; };
@@ -470,7 +462,6 @@ struct Unit<Q4MI_T_IQ4_XS> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = false;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 10;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t qs, b, k; };
     struct Raw { u32x4_t q[2]; u32x2_t h; };    // h: d | scales_h, scales_l
@@ -511,7 +502,6 @@ struct Unit<Q4MI_T_Q6_K> {
     static constexpr uint32_t kTabBytes = 0;
     static constexpr bool kTwo = true;
     static constexpr bool kOneD = true;
-    static constexpr int kRegs = 21;
     static constexpr bool kRawW = false;
     struct Offs { uint32_t ql, qh, sc, d, s, ss, b; };
     struct Raw { u32x4_t l[2], h[2]; uint32_t l8, h8; u32x2_t sc; uint32_t d; };

@@ -21,10 +21,8 @@ hipStream_t stream();
 // illegal inside a graph capture; q4_hip_moe_scratch_warm / q4_mmvq_warm
 // size everything up front.
 struct Scratch {
-    float *pd = nullptr;        // MoE decode partials [64][8][n_embd]
+    float *pd = nullptr;        // decode h [64 unique experts][8 tokens][n_ff]
     size_t pd_floats = 0;
-    uint32_t *tickets = nullptr;  // per-row-tile completion counters
-    size_t n_tickets = 0;
     int8_t *xq = nullptr;       // q8 activations for q4_mmvq_n
     float *xd = nullptr;
     size_t xq_elems = 0;
@@ -32,7 +30,7 @@ struct Scratch {
 Scratch &lib_scratch();
 
 // Grow policy of every library scratch buffer that a captured graph can
-// reference (decode partials, GEMV activations, MMQ tile list, pack
+// reference (decode h, GEMV activations, MMQ tile list, pack
 // histograms):
 //   - no growth while the library stream is being captured: an allocation
 //     there would not replay, so the call fails with GrowCapturing and the
@@ -67,7 +65,6 @@ bool stream_capturing();
 uint32_t mmq_status(int clear);
 
 bool ensure_pd(size_t floats);
-bool ensure_tickets(size_t n);
 bool ensure_xq(size_t elems);
 
 // route_k launch writing per-token lists (route.hip): row t at t*ostride,

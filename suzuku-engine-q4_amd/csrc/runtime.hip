@@ -1,6 +1,5 @@
 // Library runtime: stream selection, device scratch and error text.
 #include <stdarg.h>
-#include <string.h>
 
 #include "q4mi_internal.h"
 
@@ -56,17 +55,6 @@ bool ensure_pd(size_t floats) {
     if (g_scr.pd_floats >= floats) return true;
     if (!grow((void **)&g_scr.pd, floats * sizeof(float), "pd")) return false;
     g_scr.pd_floats = floats;
-    return true;
-}
-
-bool ensure_tickets(size_t n) {
-    if (g_scr.n_tickets >= n) return true;
-    // The counters must start at zero; every kernel that uses them returns
-    // them to zero before it exits.
-    if (!grow((void **)&g_scr.tickets, n * sizeof(uint32_t), "tickets")) return false;
-    if (hipMemset(g_scr.tickets, 0, n * sizeof(uint32_t)) != hipSuccess) return false;
-    if (hipDeviceSynchronize() != hipSuccess) return false;
-    g_scr.n_tickets = n;
     return true;
 }
 
@@ -149,21 +137,15 @@ int q4mi_per_device_selftest(void) {
 #endif
 
 const char *q4mi_status_text(uint32_t bits) {
-    static char buf[384];
+    static char buf[256];
     if (!bits) return "ok";
     if (bits & 0x80000000u) return "device status not readable";
-    buf[0] = 0;
-    if (bits & 3u)
-        snprintf(buf, sizeof buf, "decode kernel gave up a bounded wait (%s%s%s): results of the "
-                 "calls since the last status check are wrong",
-                 (bits & 1u) ? "consumer" : "", (bits & 3u) == 3u ? ", " : "",
-                 (bits & 2u) ? "producer" : "");
-    if (bits & 4u) {
-        const size_t l = strlen(buf);
-        snprintf(buf + l, sizeof buf - l, "%sXG tile record out of range (rows outside 1..128 or "
-                 "a negative slot or row): that tile was skipped, its rows not written",
-                 l ? "; " : "");
-    }
+    const char *xg = "XG tile record out of range (rows outside 1..128 or a negative slot or row): "
+                     "that tile was skipped, its rows not written";
+    const uint32_t other = bits & ~4u;
+    if (!other) return xg;
+    snprintf(buf, sizeof buf, "%s%sunknown status bits 0x%x", bits & 4u ? xg : "",
+             bits & 4u ? "; " : "", other);
     return buf;
 }
 

@@ -306,5 +306,5 @@ def test_moe_wide_hidden(gpu, oracle, n_embd, n_tok):
 
 
 def test_device_status_clean(gpu):
-    """After the decode tests, no bounded in-kernel wait gave up."""
+    """After the decode tests, no kernel has anything to report."""
     assert gpu.q4mi_device_status(1) == 0, q4mi.last_error()
