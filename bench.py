@@ -1018,8 +1018,8 @@ def bench_gemv(L, torch, np, q4mi, synth, ty, rows, K, copies, nt, label, reps=3
             "GB/s": round(nbytes / t / 1e9, 1),
             "pct_of_hbm": round(100 * nbytes / t / 1e9 / HBM_PEAK, 2),
             "us_eager": round(t_eager * 1e6, 2),
-            "note": "fp32 x in, q8 quantization included (inside the GEMV blocks for <= 1024 "
-                    "row tiles, else one quantize launch); us = graph replay of the %d "
+            "note": "fp32 x in, q8 quantization included (inside the GEMV blocks, or one launch "
+                    "ahead of a tall Q8_0 matrix at one token); us = graph replay of the %d "
                     "back-to-back calls over distinct weight copies, us_eager = the same "
                     "calls launched eagerly from Python" % copies}
 

@@ -297,17 +297,17 @@ __device__ inline double silu_mul(double g, double u) {
 // launch itself (1.7 us), the prologue (activations in, q8 codes and tables
 // in LDS, 1.6 us) and one burst of weights with its decode behind it; a
 // window's is its table lookups (random LDS banks), the decode's VALU and the
-// L1 path in about equal parts.  Measured per launch, copying rows through an
-// LDS ring / this kernel: one token 7.1 / 6.6 us, 4 tokens (36 MB) 16.8 / 13.0
-// us, 4 tokens at hidden 2560 IQ2_S (43 MB) 24.6 / 19.8 us.
+// L1 path in about equal parts.  Measured per launch (kernel trace), copying rows
+// through an LDS ring / this kernel: one token 7.1 / 6.7 us, 4 tokens (36 MB)
+// 16.8 / 13.0 us, 4 tokens at hidden 2560 IQ2_S (43 MB) 24.6 / 19.5 us.
 // One block of 16 waves per CU: two blocks of 64-register waves repeat the
 // prologue and took 19.0 us for the 4-token launch.
 //
 // Sums and silu are taken in fp64, at fp32's instruction rate: h is then the
 // correctly rounded one but for about 1e-9 of it, so that its q8 codes in the
 // down launch, which an fp32 sum's error moves now and then (about one code in
-// 200,000), are those of exact arithmetic.  (The times above are with fp32 sums;
-// fp64 adds 0.2 us at one token and 0.3 to 0.9 at four.)
+// 200,000), are those of exact arithmetic.  fp64 adds 0.2 us at one token and
+// 0.3 to 0.9 at four, which the times above include.
 //
 // A wave's task is RPW = 64 / LPR intermediate rows of one expert: LPR lanes
 // per row with UPL units each (unit li + LPR m), first the gate rows, then
@@ -529,9 +529,9 @@ __global__ __launch_bounds__(kT) void moe_gu_k(MoeArgs a) {
 // ---------------------------------------------------------------- down
 // What bounds it: the prologue (every block quantizes every selected h row)
 // and, behind it, the weights' decode as above.  Measured per launch, copying
-// rows through an LDS ring / this kernel: one token 6.6 / 5.0 us, 4 tokens
-// (hidden 2048, 18 MB) 15.9 / 9.6 us, 4 tokens at hidden 2560 IQ4_NL 20.8 /
-// 14.8 us.
+// rows through an LDS ring / this kernel: one token 6.6 / 4.9 us, 4 tokens
+// (hidden 2048, 18 MB) 15.9 / 9.1 us, 4 tokens at hidden 2560 IQ4_NL 20.8 /
+// 14.5 us.
 //
 // A block owns dn_rows output rows.  Its waves form dn_rows / (rows per wave)
 // row slices; the waves of a slice take every kES-th expert each, their lanes

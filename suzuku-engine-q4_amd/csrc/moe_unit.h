@@ -13,7 +13,9 @@
 // wave instruction over consecutive units: dwordx4 at 2-byte offsets 56-72
 // accesses, at 4-byte offsets 22-28; dword 56-62 against 14).  So every field
 // is loaded as the whole dwords around it and shifted into place by the
-// lane's byte shift: 110 instead of 266 accesses per IQ3_S wave unit.
+// lane's byte shift: 110 instead of 266 accesses per IQ3_S wave unit, adding
+// those counts up (a 4-token gate/up launch as a whole, its activations, tables,
+// stores and last refills included, has 163 per wave unit).
 //
 // Unit<TY>:
 //   Offs          the dword offsets of the lane's fields from a uniform base
