@@ -49,7 +49,7 @@ __global__ __launch_bounds__(NTHR) void mmvq_k(const uint8_t *__restrict__ W, ui
     // operations complete in issue order, so loads issued behind the copies
     // return when the copies have landed (measured: copies first, or copies
     // from fewer waves while the others build the table and quantize, are
-    // slower for configs[0]).
+    // slower for IQ3_S 4096 x 4096).
     Q4MI_GTR(0);
     F::init(tab, tid, NTHR);
     Q4MI_GTR(1);
@@ -433,7 +433,7 @@ static bool mmvq_launch_nt(const uint8_t *W, uint32_t rows, uint32_t K, const fl
     // (one row per wave) while that still fills the CUs, else 512 threads
     // per 512 / tpr rows.  The compute after a tile lands is then a quarter
     // (a half) of a 256-thread block's, whose waves take four rows each
-    // (configs[0]: 256 blocks of 16 rows, 6.2 against 7.1 us).  Several
+    // (IQ3_S 4096 x 4096: 256 blocks of 16 rows, 6.2 against 7.1 us).  Several
     // tokens' x registers fit 1024-thread blocks (128 VGPRs) only at one
     // token, 512-thread blocks up to two.
     if (xf && L.tpr) {
@@ -448,7 +448,7 @@ static bool mmvq_launch_nt(const uint8_t *W, uint32_t rows, uint32_t K, const fl
         }
     }
     // pre-quantized x at one token (the tall matrices, many tiles per CU):
-    // 512-thread blocks of one row per wave (configs[4] n=1: 59.8 against
+    // 512-thread blocks of one row per wave (Q8_0 151936 x 2048: 59.8 against
     // 61.2 us, 8-row tiles either way)
     if (!xf && NT == 1 && L.tpr) {
         const uint32_t r = 512u / (uint32_t)L.tpr;

@@ -22,7 +22,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC",
     # Packed FP32 instructions stay off (the hardware's packed forms are not
-    # trusted on this pool); the host pass ignores the feature with a warning.
+    # trusted here); the host pass ignores the feature with a warning.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-pragmas",

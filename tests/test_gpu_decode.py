@@ -186,7 +186,7 @@ def test_q4_mmvq_n_in_block_quant(gpu, ty, K, rows, n):
 
 
 def test_config0_full(gpu, oracle):
-    """BASELINE config 0: IQ3_S 4096x4096, one token."""
+    """IQ3_S 4096x4096, one token."""
     rng = np.random.default_rng(0)
     K = rows = 4096
     w = synth.matrix(rng, T_IQ3_S, rows, K)
@@ -203,7 +203,7 @@ def test_config0_full(gpu, oracle):
 # ------------------------------------------------------------ MoE decode
 
 class Layer:
-    """A MoE layer at BASELINE config shapes: 512 routed experts + 1 shared
+    """A MoE layer at hidden 2048: 512 routed experts + 1 shared
     (slot 512), hidden 2048, expert intermediate 512, all IQ3_S."""
 
     def __init__(self, seed, n_exp=513, n_embd=2048, n_ff=512):
@@ -246,7 +246,7 @@ def routed_ids(oracle, rng, k=10, E=512):
 
 
 def test_moe_decode_config2(gpu, oracle):
-    """top-10 routed + shared expert (weight 1), 1 token."""
+    """Hidden 2048: top-10 routed + shared expert (weight 1), 1 token."""
     ly = layer()
     rng = np.random.default_rng(21)
     x = rng.standard_normal(ly.n_embd).astype(np.float32)
@@ -381,7 +381,7 @@ def test_moe_exec_dev_and_rejects(gpu, oracle):
 
 @pytest.mark.parametrize("n_tok", [2, 4, 8])
 def test_moe_window_config3(gpu, oracle, n_tok):
-    """n_tok tokens (1 accepted + drafts), each with its
+    """A verify window: n_tok tokens (1 accepted + drafts), each with its
     own top-10 + the shared expert; experts shared by tokens read once."""
     ly = layer()
     rng = np.random.default_rng(30 + n_tok)

@@ -131,7 +131,7 @@ def test_mmq_group_sums_exact(gpu, oracle):
 
 
 def test_prefill_layer_config3(gpu, oracle):
-    """BASELINE config 3-prefill: 2048 tokens, Zipf-skewed top-10 over 512
+    """2048 tokens, Zipf-skewed top-10 over 512
     experts + the shared expert; route -> stable pack -> quantize ->
     MMQ gate/up -> SwiGLU -> quantize -> MMQ down -> weighted reduce.
     Checked on a sample of tokens against the oracle's composition."""

@@ -1,8 +1,8 @@
-"""GPU parity at the BASELINE configurations' full shapes, through the C ABI,
+"""GPU parity at the benchmark's full shapes, through the C ABI,
 against the C oracle:
 
-- config 4: the Q8_0 151936 x 2048 lm-head through q4_mmvq_n, 1 and 4 tokens;
-- config 3-prefill: the fused prefill sequence the benchmark times
+- LM head: the Q8_0 151936 x 2048 lm-head through q4_mmvq_n, 1 and 4 tokens;
+- prefill: the fused prefill sequence the benchmark times
   (route, q4mi_assign, q8(x), q4mi_mmq_gate_up_x, q4mi_mmq_mul_id_x,
   q4mi_expert_reduce_x, the shared expert riding in the routed launches),
   on 288 sampled tokens including the first and the last;
@@ -113,11 +113,11 @@ def down_from_codes(oracle, arena, stride, od, H, F, ids, wts, codes, scales):
         return np.stack(list(ex.map(one, range(T))))
 
 
-# ------------------------------------------------------------ config 4
+# ------------------------------------------------------------ LM head
 
 @pytest.mark.parametrize("n", [1, 4])
 def test_config4_lmhead_full(gpu, oracle, n):
-    """BASELINE config 4 at its stated shape: Q8_0 151936 x 2048 (330 MB),
+    """The LM head at full size: Q8_0 151936 x 2048 (330 MB),
     fp32 x quantized inside q4_mmvq_n, 1 and 4 tokens."""
     import torch
     rows, K = 151936, 2048
@@ -142,10 +142,10 @@ def test_config4_lmhead_full(gpu, oracle, n):
     assert rel_err(yg, yo) <= TOL
 
 
-# -------------------------------------------------------- config 3-prefill
+# -------------------------------------------------------- prefill
 
 def test_prefill_fused_path_config3(gpu, oracle):
-    """The benchmark's prefill sequence at config 3-prefill (2048 tokens,
+    """The benchmark's prefill sequence at full size (2048 tokens,
     Zipf-skewed top-10 over 512 experts, the shared expert as expert 512 at
     weight 1 in the routed launches) against the oracle on 288 tokens; the
     q8(h) codes of every sampled (token, pick) row are counted against the
@@ -227,7 +227,7 @@ def test_prefill_fused_path_config3(gpu, oracle):
 
 def test_decode_h_codes(gpu, oracle):
     """The decode layer's fp32 h (read back with q4mi_moe_copy_h) against the
-    oracle's h over 20 config-2 seeds: h within 1e-5 of each row's scale;
+    oracle's h over 20 seeds at hidden 2048: h within 1e-5 of each row's scale;
     q8(h) codes equal to the oracle's on all but <= 1e-4 of the values; y
     equal to the oracle's down path fed with the GPU's own q8(h) on every
     seed, and to the oracle end to end on every seed without a flipped code."""
